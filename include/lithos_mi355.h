@@ -457,7 +457,7 @@ typedef struct mi_sample_desc {
   uint32_t step;
   const mi_step_state* state; /* optional: seed and step from the step state */
   void* workspace;            /* optional, mi_sample_workspace_bytes, zeroed once before its first use (the
-                                 histograms and counters are left at zero by every call); NULL: the library's own */
+                                 arrival counters are left at zero by every call); NULL: the library's own */
   size_t workspace_bytes;
 } mi_sample_desc;
 size_t mi_sample_workspace_bytes(const mi_sample_desc* d);

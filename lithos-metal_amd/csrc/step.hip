@@ -5,6 +5,7 @@
 
 #include <time.h>
 
+#include <algorithm>
 #include <chrono>
 #include <deque>
 #include <mutex>
@@ -38,11 +39,16 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
 
 // The order "larger value, then lower index" over the numbers is total, so combining partial results in any order
 // gives the same answer: the spans of a row run in parallel and the last one to finish folds them.
-constexpr int ARGMAX_SPAN = ARGMAX_THREADS * 16;   // logits per workgroup
-constexpr int ARGMAX_MAX_SPANS = 256;
+constexpr int ARGMAX_SPAN = ARGMAX_THREADS * 8;    // logits per workgroup
+constexpr int ARGMAX_MAX_SPANS = 512;
 constexpr size_t ARGMAX_COUNTERS = 256;            // bytes: 16 per-row arrival counters, padded
 
-struct ArgmaxPartial { float v; int i; };
+__device__ __forceinline__ void st_dev8(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_dev8(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 __device__ __forceinline__ void block_best(float& bv, int& bi, float* sv, int* si) {
   for (int o = 32; o > 0; o >>= 1) {
@@ -64,7 +70,7 @@ __device__ __forceinline__ void block_best(float& bv, int& bi, float* sv, int* s
 // splitmix64 hash of (seed, step, token row, index): the reference's counter-based noise, so a draw is reproducible
 // bit for bit and checkable against the host restatement.
 struct SampleCtx {
-  const float* tau;                // per row: the logit threshold (select_thresholds)
+  const float* tau;                // per row: the logit threshold (sample_threshold); null: keep every logit
   float inv_t;
   uint32_t seed_lo, seed_hi, step;
   const mi_step_state* st;         // when set: seed = (rng_hi, rng_lo) and step come from the step state
@@ -92,26 +98,11 @@ constexpr uint32_t HIST_KEYS = 65536;
 constexpr int SELECT_THREADS = 1024;
 constexpr int SELECT_WAVES = SELECT_THREADS / 64;
 constexpr uint32_t WAVE_KEYS = HIST_KEYS / SELECT_WAVES;   // keys per wave, descending from 65535 − 4096·w
+constexpr int KEY_BLOCK = 64;                              // keys a thread counts and merges (1024 blocks)
+constexpr int PART_U64 = KEY_BLOCK * 2 / 8;                // a block's 16-bit counts, in 8-byte words
+constexpr int SELECT_MIN_WGS = 4;
+constexpr int SELECT_SPAN_MAX = 65528;                     // logits per workgroup: a 16-bit count cannot overflow
 
-// grid (spans, rows): the histogram of each row's logit keys (device-scope atomic adds; select clears it again)
-__global__ __launch_bounds__(ARGMAX_THREADS) void sample_hist(const uint16_t* logits, int ld, int vocab, uint32_t* hist) {
-  const int row = blockIdx.y;
-  const uint16_t* p = logits + (long long)row * ld;
-  uint32_t* h = hist + (size_t)row * HIST_KEYS;
-  const int lo = blockIdx.x * ARGMAX_SPAN, hi = min(lo + ARGMAX_SPAN, vocab);
-  for (int c = lo + (int)threadIdx.x; c < hi; c += ARGMAX_THREADS) atomicAdd(h + key16(p[c]), 1u);
-}
-
-// inclusive prefix over the 64 lanes of a wave (lane order)
-template <typename T>
-__device__ __forceinline__ T wave_scan_incl(T v, int lane) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const T u = __shfl_up(v, off);
-    if (lane >= off) v += u;
-  }
-  return v;
-}
 template <typename T>
 __device__ __forceinline__ T wave_total(T v) {
 #pragma unroll
@@ -119,65 +110,287 @@ __device__ __forceinline__ T wave_total(T v) {
   return v;
 }
 
-// the key where a descending cumulative sum starting at `run` first reaches `target`, walking this wave's keys
-// (chunks of 64, lane 0 the highest key of a chunk); -inf when the wave's keys do not get there
-template <bool MASS>
-__device__ float walk_to(const uint32_t* h, uint32_t hi, float vmax, float inv_t, double run_in, double target, int lane) {
-  float run = (float)run_in;
-  float last = -INFINITY;                           // the lowest key with a count walked so far
-  for (int q = 0; q < WAVE_KEYS / 64; ++q) {
-    const uint32_t k = hi - 64 * q - lane;
-    const uint32_t cnt = h[k];
-    const float x = MASS ? (cnt ? (float)cnt * expf((key_val(k) - vmax) * inv_t) : 0.0f) : (float)cnt;
-    const float incl = run + wave_scan_incl(x, lane);
-    const unsigned long long hit = __ballot(cnt != 0u && incl >= (float)target);
-    if (hit) return key_val(hi - 64 * q - (uint32_t)__builtin_ctzll(hit));
-    const unsigned long long nz = __ballot(cnt != 0u);
-    if (nz) last = key_val(hi - 64 * q - (63u - (uint32_t)__builtin_clzll(nz)));
-    run = __shfl(incl, 63);
+// A row's counts as sample_threshold's last workgroup holds them: 16 bits a key in LDS, and the few carries past them
+// (at most vocab / 65536: keys that hold more than 65535 logits)
+constexpr int MAX_CARRY = 16;
+struct KeyCounts {
+  const uint16_t* h;
+  const uint32_t* carry_key;
+  const uint32_t* carry;
+  int n_carry;
+  __device__ __forceinline__ uint32_t operator()(uint32_t k) const {
+    uint32_t c = h[k];
+    for (int i = 0; i < n_carry; ++i) c += carry_key[i] == k ? carry[i] << 16 : 0u;
+    return c;
   }
-  return last;                                      // the sums' order left the target a rounding short: the last key
+};
+
+// The chunks of 64 keys of a wave (lane 0 the highest key of a chunk) that hold a count, from the top, four at a time:
+// f(q[4], cnt[4], n) for the next n chunks (past n: chunk 63, its count taken as 0); f returns whether to stop
+template <typename F>
+__device__ __forceinline__ void for_chunks(const KeyCounts& kc, unsigned long long occ, uint32_t hi, int lane, F f) {
+  while (occ) {
+    int q[4], n = 0;
+    uint32_t c[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      q[j] = occ ? __builtin_ctzll(occ) : 63;
+      n += occ ? 1 : 0;
+      occ &= occ - 1;                               // 0 stays 0
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = kc(hi - 64 * q[j] - lane);
+#pragma unroll
+    for (int j = 1; j < 4; ++j) c[j] = j < n ? c[j] : 0u;
+    if (f(q, c)) return;
+  }
 }
 
-// one workgroup per row (sample.metal `sample_select`): wave w owns the keys 65535 − 4096·w − [0, 4096), walked
-// 64 at a time from the top (lane = key), so wave order is descending key order. tau = the most restrictive of
+// the key where a descending cumulative sum starting at `run` first reaches `target`, walking this wave's keys; -inf
+// when it has none, the lowest when the sums' order leaves the target a rounding short. A chunk's total (a balanced
+// tree over the lanes, as lane 63 of its inclusive prefix) moves the sum on; only a chunk that may hold the target (a
+// margin of 2^-16 covers the prefix's other order of the same sum) has its prefix formed, through the lane exchanges
+template <bool MASS>
+__device__ __forceinline__ float walk_to(const KeyCounts& kc, unsigned long long occ, uint32_t hi, float vmax, float inv_t,
+                                         float run, float target, int lane) {
+  float res = -INFINITY;
+  for_chunks(kc, occ, hi, lane, [&](const int (&q)[4], const uint32_t (&c)[4]) {
+    float x[4], tot[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t k = hi - 64 * q[j] - lane;
+      x[j] = MASS ? (c[j] ? (float)c[j] * expf((key_val(k) - vmax) * inv_t) : 0.0f) : (float)c[j];
+      tot[j] = wave_sum(x[j]);
+    }
+    for (int j = 0; j < 4; ++j) {
+      const float xj = j == 0 ? x[0] : j == 1 ? x[1] : j == 2 ? x[2] : x[3];
+      const float tj = j == 0 ? tot[0] : j == 1 ? tot[1] : j == 2 ? tot[2] : tot[3];
+      const uint32_t cj = j == 0 ? c[0] : j == 1 ? c[1] : j == 2 ? c[2] : c[3];
+      const uint32_t top = hi - 64 * (j == 0 ? q[0] : j == 1 ? q[1] : j == 2 ? q[2] : q[3]);
+      const unsigned long long nz = __ballot(cj != 0u);
+      if ((run + tj) * (1.0f + 1.0f / 65536.0f) >= target) {
+        float s = xj;
+        for (int off = 1; off < 64; off <<= 1) {    // inclusive prefix over the lanes
+          const float u = __shfl_up(s, off);
+          s = lane >= off ? s + u : s;
+        }
+        const unsigned long long hit = __ballot(cj != 0u && run + s >= target);
+        if (hit) {
+          res = key_val(top - (uint32_t)__builtin_ctzll(hit));
+          return true;
+        }
+      }
+      if (nz) res = key_val(top - (63u - (uint32_t)__builtin_clzll(nz)));   // the lowest key with a count so far
+      run += tj;
+    }
+    return false;
+  });
+  return res;
+}
+
+// grid (workgroups, rows): the threshold tau of each row (sample.metal `sample_select`), the most restrictive of
 // top-k (the k-th largest logit, ties kept), top-p (the key at which the descending cumulative softmax mass of
 // logits / temperature first reaches p of the total — of the top-k set's mass with flag 8) and min-p (max +
-// temperature · log(min_p)). Per-wave sums (fixed lane order), then a sequential sum over the waves decides which
-// wave walks to the key; the row's histogram is cleared after.
-__global__ __launch_bounds__(SELECT_THREADS) void sample_select(uint32_t* hist, float* tau, int top_k, float temperature,
-                                                                float top_p, float min_p, uint32_t flags) {
+// temperature · log(min_p)), from the counts of the row's logit keys.
+//
+// What bounds it is latency: half a megabyte of logits, but 65536 counters. Counting with device-scope atomics on a
+// table in memory took 88 us for a row of 248320 logits (hot keys serialize at the coherence point) and walking that
+// table from one workgroup 49 us. Here a workgroup counts its span in LDS, 16 bits a key (128 KB, so a span stays under
+// 65536 logits; at least four workgroups a row, so that counting is short), publishes the blocks of 64 keys that hold
+// anything with a 1024-bit map of them (device-scope stores), and the row's last workgroup to arrive adds the published
+// blocks to its own and finds tau, looking only at the chunks of keys that hold a count: 20 us for that row (counting
+// 6, publishing and arriving 5, merging 3, the sums and the walk 6), and 49 us with the draw for 16 rows. Six or eight
+// workgroups a row count faster and merge slower (27 us with the draw either way at 248320 logits, 21 → 23 us at 32000).
+// Every loop over the keys is rolled: with the counts in registers the kernel was 93 KB of straight-line code, and
+// fetching it cost more than its work.
+//
+// The sums keep one fixed order: wave w owns the keys 65535 − 4096·w − [0, 4096), lane l the keys ≡ 63 − l mod 64,
+// added from the top down; lanes, then waves; the wave whose share crosses the target walks its keys in order.
+__global__ __launch_bounds__(SELECT_THREADS) void sample_threshold(const uint16_t* logits, int ld, int vocab, int span,
+                                                                   uint32_t* counters, unsigned long long* maps,
+                                                                   unsigned long long* part, float* tau, int top_k,
+                                                                   float temperature, float top_p, float min_p,
+                                                                   uint32_t flags) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t h16[];   // [32768]: the counts of keys 2i, 2i + 1
   __shared__ uint32_t wmax[SELECT_WAVES];
   __shared__ uint32_t wcnt[SELECT_WAVES];
   __shared__ float wmass[SELECT_WAVES], wmass_k[SELECT_WAVES];
   __shared__ float res[2];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, row = blockIdx.x;
-  uint32_t* h = hist + (size_t)row * HIST_KEYS;
-  const uint32_t hi = HIST_KEYS - 1 - (uint32_t)w * WAVE_KEYS;
-  uint32_t km = 0;
-  for (int q = 0; q < WAVE_KEYS / 64; ++q) {
-    const uint32_t k = hi - 64 * q - lane;
-    if (h[k]) km = max(km, k);
-  }
+  __shared__ int last;
+  __shared__ uint32_t carry_key[MAX_CARRY], carry[MAX_CARRY], n_carry;
+  const int tid = threadIdx.x, lane = tid & 63, row = blockIdx.y, nb = gridDim.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lo = blockIdx.x * span, n = min(span, vocab - lo);     // n >= 1
+  const uint16_t* p = logits + (long long)row * ld + lo;
+
+  // ---- count this span ------------------------------------------------------------------------------------------
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) km = max(km, (uint32_t)__shfl_xor((int)km, off));
+  for (int i = 0; i < (int)HIST_KEYS / 2 / 4 / SELECT_THREADS; ++i)
+    reinterpret_cast<uint4*>(h16)[i * SELECT_THREADS + tid] = uint4{0u, 0u, 0u, 0u};
+  if (tid == 0) n_carry = 0;
+  __syncthreads();
+  auto count = [&](uint32_t bits) {
+    const uint32_t k = key16(bits);
+    atomicAdd(&h16[k >> 1], (k & 1u) ? 0x10000u : 1u);
+  };
+  const int nv = (reinterpret_cast<uintptr_t>(p) & 15) == 0 ? n / 8 : 0;   // whole 16-byte vectors of an aligned row
+  constexpr int UN = 4;                                                    // vectors in flight per thread
+  for (int v0 = tid; v0 < nv; v0 += UN * SELECT_THREADS) {
+    uint4 q[UN];
+#pragma unroll
+    for (int i = 0; i < UN; ++i) q[i] = reinterpret_cast<const uint4*>(p)[min(v0 + i * SELECT_THREADS, nv - 1)];
+#pragma unroll
+    for (int i = 0; i < UN; ++i) {
+      if (v0 + i * SELECT_THREADS >= nv) break;
+      const uint32_t qw[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        count(qw[e] & 0xFFFFu);
+        count(qw[e] >> 16);
+      }
+    }
+  }
+  for (int c = 8 * nv + tid; c < n; c += 8 * SELECT_THREADS) {             // the rest, or an unaligned row
+    uint16_t b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) b[i] = p[min(c + i * SELECT_THREADS, n - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (c + i * SELECT_THREADS < n) count(b[i]);
+  }
+  __syncthreads();
+
+  if (nb > 1) {
+    // ---- publish: thread b the block of keys 64·b .. + 63, its 16 words in an order rotated by the thread (no bank
+    // conflicts; the thread of the same number adds them in the same order), word i of every block side by side
+    unsigned long long* mine = reinterpret_cast<unsigned long long*>(h16) + tid * PART_U64;
+    const long long at = (long long)row * nb + blockIdx.x;
+    unsigned long long any = 0, v[PART_U64];
+#pragma unroll
+    for (int i = 0; i < PART_U64; ++i) any |= v[i] = mine[(i + tid) & (PART_U64 - 1)];
+    if (any) {
+      unsigned long long* dst = part + at * PART_U64 * SELECT_THREADS + tid;
+#pragma unroll
+      for (int i = 0; i < PART_U64; ++i) st_dev8(dst + i * SELECT_THREADS, v[i]);
+    }
+    const unsigned long long map = __ballot(any != 0);
+    if (lane == 0) st_dev8(maps + at * SELECT_WAVES + w, map);
+    // every wave's stores acknowledged at the coherence point before the row's count moves
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const uint32_t prev = __hip_atomic_fetch_add(counters + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = prev == (uint32_t)(nb - 1);
+      if (last) __hip_atomic_store(counters + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last) return;
+
+    // ---- the row's last workgroup: add the other workgroups' blocks, three workgroups at a time. Wave w adds word w of
+    // the blocks; it goes through the groups of 64 blocks that any of the three holds, four groups' loads in flight. A
+    // block its map leaves out was not written: read, and not added
+    constexpr int MG = 3, BG = 4;
+    static_assert(SELECT_WAVES == PART_U64, "wave w adds word w of every block");
+    auto wg_of = [&](int i) { return (long long)row * nb + (blockIdx.x + 1 + i) % nb; };   // the others, i < nb − 1
+    for (int g0 = 0; g0 < nb - 1; g0 += MG) {
+      unsigned long long m[MG], held = 0;              // lane l: the maps' words of blocks 64·(l % 16) .. + 63
+#pragma unroll
+      for (int g = 0; g < MG; ++g) m[g] = ld_dev8(maps + wg_of(min(g0 + g, nb - 2)) * SELECT_WAVES + (lane & 15));
+#pragma unroll
+      for (int g = 0; g < MG; ++g) {
+        if (g0 + g >= nb - 1) m[g] = 0;                // past the last: re-read, not added
+        held |= m[g];
+      }
+      uint32_t todo = (uint32_t)__ballot(held != 0) & 0xFFFFu;
+      while (todo) {
+        unsigned long long buf[BG][MG];
+        int bg[BG], nbg = 0;
+#pragma unroll
+        for (int j = 0; j < BG; ++j) {                 // past the last group: the group before again, not added
+          if (todo) { bg[j] = __builtin_ctz(todo); ++nbg; } else { bg[j] = bg[max(j - 1, 0)]; }
+          todo &= todo - 1;
+#pragma unroll
+          for (int g = 0; g < MG; ++g)
+            buf[j][g] = ld_dev8(part + (wg_of(min(g0 + g, nb - 2)) * PART_U64 + w) * SELECT_THREADS + 64 * bg[j] + lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < BG; ++j) {
+          if (j >= nbg) break;
+          unsigned long long x[MG];
+#pragma unroll
+          for (int g = 0; g < MG; ++g) {
+            const unsigned long long on = (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)m[g], bg[j]) |
+                                          ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(m[g] >> 32), bg[j]) << 32);
+            x[g] = (on >> lane) & 1ull ? buf[j][g] : 0ull;
+          }
+          const int b = 64 * bg[j] + lane, word = b * PART_U64 + ((w + b) & (PART_U64 - 1));
+          unsigned long long* at64 = reinterpret_cast<unsigned long long*>(h16) + word;
+          const unsigned long long own = *at64;
+          uint32_t c[4] = {(uint32_t)own & 0xFFFFu, (uint32_t)own >> 16, (uint32_t)(own >> 32) & 0xFFFFu, (uint32_t)(own >> 48)};
+#pragma unroll
+          for (int g = 0; g < MG; ++g) {
+            c[0] += (uint32_t)x[g] & 0xFFFFu;
+            c[1] += (uint32_t)x[g] >> 16;
+            c[2] += (uint32_t)(x[g] >> 32) & 0xFFFFu;
+            c[3] += (uint32_t)(x[g] >> 48);
+          }
+          *at64 = (unsigned long long)((c[0] & 0xFFFFu) | (c[1] << 16)) |
+                  ((unsigned long long)((c[2] & 0xFFFFu) | (c[3] << 16)) << 32);
+          if ((c[0] | c[1] | c[2] | c[3]) >> 16) {     // a key past 65535
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (c[e] >> 16) {
+                const uint32_t slot = atomicAdd(&n_carry, 1u);
+                if (slot < MAX_CARRY) { carry_key[slot] = 4 * word + e; carry[slot] = c[e] >> 16; }
+              }
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  // ---- tau: thread (w, l) takes the keys hi − 64·q − l, hi = 65535 − 4096·w; occ: the chunks q that hold a count -----
+  const KeyCounts kc{reinterpret_cast<const uint16_t*>(h16), carry_key, carry, (int)min(n_carry, (uint32_t)MAX_CARRY)};
+  const uint32_t hi = HIST_KEYS - 1 - (uint32_t)w * WAVE_KEYS;
+  unsigned long long occ = 0;
+  for (int q0 = 0; q0 < 64; q0 += 16) {
+    uint32_t c[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) c[j] = kc.h[hi - 64 * (q0 + j) - lane];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) occ |= __ballot(c[j] != 0u) ? 1ull << (q0 + j) : 0ull;
+  }
+  if (kc.n_carry)                                   // a count of 65536, …: its low bits may be 0
+    for (int i = 0; i < kc.n_carry; ++i)
+      if (carry_key[i] <= hi && carry_key[i] > hi - WAVE_KEYS) occ |= 1ull << ((hi - carry_key[i]) >> 6);
+  uint32_t km = 0;                                  // the wave's highest key with a count
+  if (occ) {
+    const uint32_t top = hi - 64 * (uint32_t)__builtin_ctzll(occ);
+    km = top - (uint32_t)__builtin_ctzll(__ballot(kc(top - lane) != 0u));
+  }
   if (lane == 0) wmax[w] = km;
-  if (threadIdx.x == 0) { res[0] = -INFINITY; res[1] = -INFINITY; }
+  if (tid == 0) { res[0] = -INFINITY; res[1] = -INFINITY; }
   __syncthreads();
   uint32_t gmax = 0;
+#pragma unroll
   for (int i = 0; i < SELECT_WAVES; ++i) gmax = max(gmax, wmax[i]);
   const float vmax = key_val(gmax), inv_t = 1.0f / temperature;
   float tau_k = -INFINITY, tau_p = -INFINITY, tau_m = -INFINITY;
   if (flags & 1u) {                                 // top-k: counts are exact
-    uint32_t cnt = 0;
-    for (int q = 0; q < WAVE_KEYS / 64; ++q) cnt += h[hi - 64 * q - lane];
-    cnt = wave_total(cnt);
-    if (lane == 0) wcnt[w] = cnt;
+    uint32_t c = 0;
+    for_chunks(kc, occ, hi, lane, [&](const int (&)[4], const uint32_t (&x)[4]) {
+      c += x[0] + x[1] + x[2] + x[3];
+      return false;
+    });
+    c = wave_total(c);
+    if (lane == 0) wcnt[w] = c;
     __syncthreads();
     uint32_t before = 0;
     for (int i = 0; i < w; ++i) before += wcnt[i];
     if (before < (uint32_t)top_k && before + wcnt[w] >= (uint32_t)top_k) {
-      const float kk = walk_to<false>(h, hi, vmax, inv_t, (double)before, (double)top_k, lane);
+      const float kk = walk_to<false>(kc, occ, hi, vmax, inv_t, (float)before, (float)top_k, lane);
       if (lane == 0) res[0] = kk;
     }
     __syncthreads();
@@ -185,15 +398,20 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_select(uint32_t* hist, 
   }
   if (flags & 2u) {
     float m = 0.0f, mk = 0.0f;
-    for (int q = 0; q < WAVE_KEYS / 64; ++q) {
-      const uint32_t k = hi - 64 * q - lane;
-      const uint32_t cnt = h[k];
-      if (cnt) {
-        const float x = (float)cnt * expf((key_val(k) - vmax) * inv_t);
-        m += x;
-        if (key_val(k) >= tau_k) mk += x;
+    for_chunks(kc, occ, hi, lane, [&](const int (&q)[4], const uint32_t (&c)[4]) {
+      float kv[4], x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        kv[j] = key_val(hi - 64 * q[j] - lane);
+        x[j] = (float)c[j] * expf((kv[j] - vmax) * inv_t);
       }
-    }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        m = c[j] ? m + x[j] : m;
+        mk = c[j] && kv[j] >= tau_k ? mk + x[j] : mk;
+      }
+      return false;
+    });
     m = wave_total(m);
     mk = wave_total(mk);
     if (lane == 0) { wmass[w] = m; wmass_k[w] = mk; }
@@ -203,19 +421,14 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_select(uint32_t* hist, 
     for (int i = 0; i < w; ++i) before += wmass[i];
     const float target = top_p * total;
     if (before < target && before + wmass[w] >= target) {
-      const float kp = walk_to<true>(h, hi, vmax, inv_t, (double)before, (double)target, lane);
+      const float kp = walk_to<true>(kc, occ, hi, vmax, inv_t, before, target, lane);
       if (lane == 0) res[1] = kp;
     }
     __syncthreads();
     tau_p = res[1];
   }
   if (flags & 4u) tau_m = vmax + temperature * logf(min_p);
-  if (threadIdx.x == 0) tau[row] = fmaxf(fmaxf(tau_k, tau_p), tau_m);
-  __syncthreads();                                  // every wave's reads before the clearing stores
-  for (int q = 0; q < WAVE_KEYS / 64; ++q) {
-    const uint32_t k = hi - 64 * q - lane;
-    if (h[k]) h[k] = 0u;                            // clear for the next call
-  }
+  if (tid == 0) tau[row] = fmaxf(fmaxf(tau_k, tau_p), tau_m);
 }
 
 // grid (spans, rows): each workgroup scans ARGMAX_SPAN logits of one row with 16-byte loads, publishes its best,
@@ -223,7 +436,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_select(uint32_t* hist, 
 // value of a BF16 logit v >= tau is v / temperature + its Gumbel noise, any other logit is left out.
 template <bool SAMPLE>
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_spans(mi_argmax_desc d, uint32_t* counters,
-                                                               ArgmaxPartial* part, SampleCtx sc) {
+                                                               unsigned long long* part, SampleCtx sc) {
   __shared__ float sv[ARGMAX_THREADS / 64];
   __shared__ int si[ARGMAX_THREADS / 64];
   __shared__ int last;
@@ -234,7 +447,7 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_spans(mi_argmax_desc d,
   float th = 0.0f;
   uint32_t seed_lo = 0, seed_hi = 0, step = 0;
   if constexpr (SAMPLE) {
-    th = sc.tau[row];
+    th = sc.tau ? sc.tau[row] : -INFINITY;          // null: every logit kept
     seed_lo = sc.st ? (uint32_t)sc.st->rng_lo : sc.seed_lo;
     seed_hi = sc.st ? (uint32_t)sc.st->rng_hi : sc.seed_hi;
     step = sc.st ? sc.st->step : sc.step;
@@ -280,25 +493,29 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_spans(mi_argmax_desc d,
     }
   }
   block_best(bv, bi, sv, si);
+  // published without a fence (an agent-scope release writes back the whole L2): the partial's device-scope store is
+  // acknowledged before the row's count moves, and the last workgroup reads the partials with device-scope loads
   if (tid == 0) {
-    part[row * nb + blockIdx.x] = ArgmaxPartial{bv, bi};
-    __threadfence();
-    last = atomicAdd(&counters[row], 1u) == (uint32_t)(nb - 1);
+    st_dev8(part + row * nb + blockIdx.x,
+            (unsigned long long)__float_as_uint(bv) | ((unsigned long long)(uint32_t)bi << 32));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(&counters[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(nb - 1);
   }
   __syncthreads();
   if (!last) return;
-  __threadfence();
   bv = -INFINITY;
   bi = 0x7FFFFFFF;
   for (int k = tid; k < nb; k += ARGMAX_THREADS) {
-    const ArgmaxPartial q = part[row * nb + k];
-    if (better(q.v, q.i, bv, bi)) { bv = q.v; bi = q.i; }
+    const unsigned long long q = ld_dev8(part + row * nb + k);
+    const float qv = __uint_as_float((uint32_t)q);
+    const int qi = (int)(uint32_t)(q >> 32);
+    if (better(qv, qi, bv, bi)) { bv = qv; bi = qi; }
   }
   __syncthreads();                                  // sv / si are reused
   block_best(bv, bi, sv, si);
   if (tid == 0) {
     d.ids[row] = bi == 0x7FFFFFFF ? -1 : bi;        // no number in the row
-    atomicExch(&counters[row], 0u);
+    __hip_atomic_store(&counters[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -345,8 +562,12 @@ __global__ __launch_bounds__(64) void advance_step(mi_advance_desc d) {
 
 int argmax_spans_of(int vocab) { return (vocab + ARGMAX_SPAN - 1) / ARGMAX_SPAN; }
 
-__global__ void fill_neg_inf(float* p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = -INFINITY;
+// sample_threshold's workgroups per row and the logits each counts (a multiple of 8: rows stay 16-byte aligned)
+int select_span_of(int vocab, int* wgs) {
+  const int n = std::max(SELECT_MIN_WGS, (vocab + SELECT_SPAN_MAX - 1) / SELECT_SPAN_MAX);
+  const int span = ((vocab + n - 1) / n + 7) / 8 * 8;
+  *wgs = (vocab + span - 1) / span;
+  return span;
 }
 
 __global__ __launch_bounds__(64) void verify_select_step(mi_verify_select_desc d) {
@@ -571,7 +792,7 @@ int mi_embed(const mi_embed_desc* d, void* stream) {
 
 size_t mi_argmax_workspace_bytes(const mi_argmax_desc* d) {
   if (!d || d->t < 1 || d->vocab < 1) return 0;
-  return ARGMAX_COUNTERS + (size_t)d->t * argmax_spans_of(d->vocab) * sizeof(ArgmaxPartial);
+  return ARGMAX_COUNTERS + (size_t)d->t * argmax_spans_of(d->vocab) * sizeof(unsigned long long);
 }
 
 int mi_argmax(const mi_argmax_desc* d, void* stream) {
@@ -587,25 +808,29 @@ int mi_argmax(const mi_argmax_desc* d, void* stream) {
     return rc;
   }
   auto* counters = static_cast<uint32_t*>(ws);
-  auto* part = reinterpret_cast<ArgmaxPartial*>(static_cast<char*>(ws) + ARGMAX_COUNTERS);
+  auto* part = reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + ARGMAX_COUNTERS);
   hipLaunchKernelGGL(argmax_spans<false>, dim3(nb, d->t), dim3(ARGMAX_THREADS), 0, static_cast<hipStream_t>(stream),
                      *d, counters, part, SampleCtx{});
   MI_TRY_HIP(hipGetLastError(), "argmax launch");
   return MI_OK;
 }
 
-// workspace: argmax counters | partials | tau[16] | histograms [t][65536] u32
-size_t sample_layout(int t, int vocab, size_t* off_tau, size_t* off_hist) {
-  const size_t part = ARGMAX_COUNTERS + (size_t)t * argmax_spans_of(vocab) * sizeof(ArgmaxPartial);
+// workspace: argmax counters (16, then sample_threshold's 16) | partials | tau[16] | per (row, workgroup of
+// sample_threshold): the maps of its key blocks [16] u64 | the blocks' 16-bit counts [1024][64]
+size_t sample_layout(int t, int vocab, size_t* off_tau, size_t* off_map, size_t* off_part) {
+  const size_t part = ARGMAX_COUNTERS + (size_t)t * argmax_spans_of(vocab) * sizeof(unsigned long long);
+  int wgs = 0;
+  (void)select_span_of(vocab, &wgs);
   *off_tau = (part + 255) / 256 * 256;
-  *off_hist = *off_tau + 256;
-  return *off_hist + (size_t)t * HIST_KEYS * sizeof(uint32_t);
+  *off_map = *off_tau + 256;
+  *off_part = *off_map + (size_t)t * wgs * SELECT_WAVES * sizeof(unsigned long long);
+  return *off_part + (size_t)t * wgs * SELECT_THREADS * PART_U64 * sizeof(unsigned long long);
 }
 
 size_t mi_sample_workspace_bytes(const mi_sample_desc* d) {
   if (!d || d->t < 1 || d->vocab < 1) return 0;
-  size_t a, b;
-  return sample_layout(d->t, d->vocab, &a, &b);
+  size_t a, b, c;
+  return sample_layout(d->t, d->vocab, &a, &b, &c);
 }
 
 int mi_sample(const mi_sample_desc* d, void* stream) {
@@ -615,8 +840,8 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
              "mi_sample: temperature > 0, top_k / top_p / min_p >= 0 (temperature 0 is mi_argmax)");
   const int nb = argmax_spans_of(d->vocab);
   MI_REQUIRE(nb <= ARGMAX_MAX_SPANS, "mi_sample: vocab %d exceeds %d", d->vocab, ARGMAX_MAX_SPANS * ARGMAX_SPAN);
-  size_t off_tau, off_hist;
-  const size_t need = sample_layout(d->t, d->vocab, &off_tau, &off_hist);
+  size_t off_tau, off_map, off_part;
+  const size_t need = sample_layout(d->t, d->vocab, &off_tau, &off_map, &off_part);
   void* ws = d->workspace;
   if (ws) {
     MI_REQUIRE(d->workspace_bytes >= need, "mi_sample: workspace %zu B < %zu B", d->workspace_bytes, need);
@@ -625,9 +850,8 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
   }
   char* wb = static_cast<char*>(ws);
   auto* counters = reinterpret_cast<uint32_t*>(wb);
-  auto* part = reinterpret_cast<ArgmaxPartial*>(wb + ARGMAX_COUNTERS);
+  auto* part = reinterpret_cast<unsigned long long*>(wb + ARGMAX_COUNTERS);
   auto* tau = reinterpret_cast<float*>(wb + off_tau);
-  auto* hist = reinterpret_cast<uint32_t*>(wb + off_hist);
   uint32_t flags = 0;
   if (d->top_k > 0) flags |= 1u;
   if (d->top_p > 0.0f && d->top_p < 1.0f) flags |= 2u;
@@ -635,11 +859,21 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
   if (d->topp_in_topk) flags |= 8u;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (flags & 7u) {
-    hipLaunchKernelGGL(sample_hist, dim3(nb, d->t), dim3(ARGMAX_THREADS), 0, s, d->logits, d->ld, d->vocab, hist);
-    hipLaunchKernelGGL(sample_select, dim3(d->t), dim3(SELECT_THREADS), 0, s, hist, tau, d->top_k, d->temperature,
-                       d->top_p, d->min_p, flags);
+    int wgs = 0;
+    const int span = select_span_of(d->vocab, &wgs);
+    const size_t lds = HIST_KEYS / 2 * sizeof(uint32_t);
+    static std::once_flag once;                     // more than 64 KB of dynamic LDS must be allowed once
+    std::call_once(once, [&] {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(sample_threshold),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      (void)hipGetLastError();
+    });
+    hipLaunchKernelGGL(sample_threshold, dim3(wgs, d->t), dim3(SELECT_THREADS), lds, s, d->logits, d->ld, d->vocab, span,
+                       counters + 16, reinterpret_cast<unsigned long long*>(wb + off_map),
+                       reinterpret_cast<unsigned long long*>(wb + off_part), tau, d->top_k, d->temperature, d->top_p,
+                       d->min_p, flags);
   } else {
-    hipLaunchKernelGGL(fill_neg_inf, dim3(1), dim3(64), 0, s, tau, d->t);        // nothing to cut: keep every logit
+    tau = nullptr;                                  // nothing to cut: keep every logit
   }
   mi_argmax_desc am{};
   am.t = d->t; am.vocab = d->vocab; am.logits = d->logits; am.ld = d->ld; am.f32 = 0; am.ids = d->ids;

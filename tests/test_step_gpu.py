@@ -558,3 +558,25 @@ def test_decoder_program_stop_inside_a_graph_leaves_the_state_of_the_emitted_ste
     for name in ("k_codes", "v_codes", "k_scales", "v_scales"):
         assert torch.equal(getattr(ca, name), getattr(cb, name)), f"KV cache {name} differs after the stop"
     assert int(cb.k_scales[:, 40 + emitted].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("vocab", [1, 9, 63, 65537, 262150, 300001])
+@pytest.mark.parametrize("opts", [dict(top_k=5), dict(top_p=0.7), dict(top_k=40, top_p=0.9, topp_in_topk=True)],
+                         ids=["k", "p", "kp"])
+def test_sample_threshold_spans(torch_gpu, vocab, opts):
+    """One logit, fewer logits than workgroups, spans around 65536 logits (their 16-bit counts), odd rows (unaligned
+    after the first), and every kind of row: spread, constant (one key holds all of them) and nearly all -inf."""
+    torch = torch_gpu
+    from monolith_mi355 import kernels
+    _say("sample_threshold", vocab, opts)
+    rng = np.random.default_rng(vocab)
+    rows = np.zeros((3, vocab), np.float32)
+    rows[0] = rng.standard_normal(vocab) * 3.0
+    rows[1] = -1.25
+    rows[2] = -np.inf
+    rows[2, rng.integers(0, vocab, 3)] = (1.0, 2.0, -3.0)
+    lb = to_dev_bf16(torch, rows)
+    lf = from_dev_bf16(lb)
+    for step in (0, 3):
+        tok = kernels.sample(lb, seed=77, step=step, temperature=0.8, **opts).cpu().tolist()
+        assert tok == [O.sample(lf[i], seed=77, step=step, t=i, temperature=0.8, **opts) for i in range(3)]
