@@ -192,6 +192,19 @@ __device__ __forceinline__ f16x8 int4_decode8(uint32_t dw) {
   return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
+// The same codes as F16 denormals, the nibbles where they stand: n·2^-24 (elements 0, 1, 4, 5) or 16n·2^-24 (2, 3, 6,
+// 7: their activations carry the 1/16) — exact, and five instructions for eight weights instead of eleven
+__device__ __forceinline__ f16x8 int4_decode8_denormal(uint32_t dw) {
+  const uint32_t hi = dw >> 8;
+  union { uint32_t u[4]; f16x8 h; } p;
+  p.u[0] = dw & 0x000F000Fu;
+  p.u[1] = dw & 0x00F000F0u;
+  p.u[2] = hi & 0x000F000Fu;
+  p.u[3] = hi & 0x00F000F0u;
+  return p.h;
+}
+__device__ __forceinline__ bool int4_high(int e) { return (e & 2) != 0; }   // the elements that carry 16n
+
 // FP8 E4M3: codes 2j, 2j+1 of a dword (hi: 2, 3) → exact BF16 / F16 pairs (scale 1: the tensor scale is the row's)
 __device__ __forceinline__ bf16x2 cvt_fp8x2_bf16(uint32_t dw, bool hi) {
   return hi ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(dw, 1.0f, true) : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(dw, 1.0f, false);
@@ -200,6 +213,11 @@ __device__ __forceinline__ f16x8 fp8_decode8(uint32_t d0, uint32_t d1) {
   const f16x2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, true);
   const f16x2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, false), e = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, true);
   return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, e.x, e.y};
+}
+
+__device__ __forceinline__ bf16x8 fp8_decode8_bf16(uint32_t d0, uint32_t d1) {
+  const bf16x2 a = cvt_fp8x2_bf16(d0, false), b = cvt_fp8x2_bf16(d0, true), c = cvt_fp8x2_bf16(d1, false), e = cvt_fp8x2_bf16(d1, true);
+  return bf16x8{a.x, a.y, b.x, b.y, c.x, c.y, e.x, e.y};
 }
 
 __device__ __forceinline__ int int4_perm8(int i) { return (i & 1) ? 4 + (i >> 1) : (i >> 1); }
@@ -1031,18 +1049,21 @@ void gemv_rowp(Args a) {
 // every one of them. The
 // wave's activations for those chunks stay in VGPRs for the whole launch as the F16 A operands of
 // v_mfma_f32_16x16x32_f16 (token = A row; each token power-of-two scaled into F16 range over the wave's slice;
-// normalized first when the input norm is fused); the weights are the B operand, decoded exactly to F16. Each wave
-// keeps two tiles in flight (NVFP4 / FP8; one for INT4) and issues the next as soon as one is consumed. A
+// a fused input norm runs as its own launch before, see wants_prenorm); the weights are the B operand, decoded exactly to F16. Each wave
+// keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5) and issues the next as soon
+// as one is consumed. FP8 takes BF16 operands instead (its codes are exact BF16, the activations as they are). A
 // tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to exact F16
 // integers, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
 // scaled and offset by its (scale, bias) pair with the token's Σx over the group (held per lane for the launch).
-// LDS: nw[K] (fused norm) | stat[S][16] | red[rt][S][16 tokens][16 rows].
+// LDS: (INT4: Σx [S][KW][2][16]) | red [S][row_ld floats]: a wave's activation stage, then its [rt][16 tokens][16 rows].
+constexpr int ROWM_SLD = 1024 + 16;             // bytes of a staged activation row (512 columns), padded
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 template <int FMT>
 __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   constexpr int KC = chunk_cols(FMT), KW = 512 / KC;   // a wave's slice is 512 columns: 4 NVFP4 / INT4, 8 FP8 chunks
   constexpr int SPC = KC / 32;                  // MFMA steps per chunk: the lane's KC/4 columns, 8 per step
   static_assert(FMT == FMT_NVFP4 || FMT == FMT_FP8 || FMT == FMT_INT4, "gemv_rowm: NVFP4, FP8 or INT4");
-  constexpr bool I4 = FMT == FMT_INT4;
+  constexpr bool I4 = FMT == FMT_INT4, F8 = FMT == FMT_FP8;
   constexpr int UB = I4 ? UNIT_Q : 1024;        // bytes from one chunk's codes to the next
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1059,12 +1080,42 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   const int g = lane >> 4, m_row = lane & 15;
   const uint8_t* wmat = a.w;
   auto tile_of = [&](int j) { return (int)blockIdx.x + j * G; };
-  float* nws = reinterpret_cast<float*>(smem);                                  // [K] when the norm is fused
-  float* stat = nws + (a.norm_w ? a.k : 0);                                    // [S][16]
-  float* sxl = stat + S * 16;                                                  // INT4: [S][KW][2][16]
-  float* red = sxl + (I4 ? S * KW * 2 * 16 : 0);                               // [rt][S][16][16]
+  float* sxl = reinterpret_cast<float*>(smem);                                  // INT4: [S][KW][2][16]
+  float* red = sxl + (I4 ? S * KW * 2 * 16 : 0);                               // [S][row_ld]: per wave its activation
+                                                                               // stage, then its tiles' [rt][16][16]
 
-  // ---- the first tile's weights, then the activations ------------------------------------------------------------
+  // ---- the A operands: xa[cc][s] = x[token m_row][c0·KC + cc·KC + col(g, s) + (0..7)], col(g, s) = (KC/4)·g + 8s
+  // (NVFP4 / FP8) or 32s + 8g (INT4: the codes' column order in a unit), in F16: per token, 2^-p brings the slice's max
+  // into [2^14, 2^15) (exact within 2^28 of the max). Four rows at a time: a row's slice is one coalesced 1 KiB load
+  // (lane l: columns 8l .. 8l + 7), its max one wave reduction, and only real tokens are converted; the rows then cross
+  // to the operand layout through the wave's LDS stage. (Loaded straight in the operand layout — 16 loads of 16-byte
+  // pieces, half of each 128-byte line a load — and converted there, padding rows and all, the prologue grew with M:
+  // 27B gate|up at
+  // M = 3 / 8 / 16 23.4 / 27.0 / 32.2 → 20.7 / 20.7 / 24.5 us, out_proj 11.0 / 12.2 / 14.7 → 8.2 / 9.4 / 13.2, both
+  // with the epilogue below.) The next rows are in flight while four are converted, the first eight ahead of the weights.
+  uint8_t* const stage = reinterpret_cast<uint8_t*>(red + wave * a.row_ld);
+  auto xcol = [&](int s) { return I4 ? 32 * s + 8 * g : (KC / 4) * g + 8 * s; };
+  const int ng = (cnt + 3) >> 2, cols = max(kw, 1) * KC;
+  const uint16_t* xbase = a.x + (long long)c0 * KC + min(8 * lane, cols - 8);
+  auto load4 = [&](uint4 (&x)[4], int grp) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = *reinterpret_cast<const uint4*>(xbase + (long long)min(4 * grp + r, cnt - 1) * a.ldx);
+  };
+  uint4 xr[4], xn[4], xa[KW][SPC];
+  if constexpr (F8) {
+    const uint16_t* xrow = a.x + (long long)min(m_row, cnt - 1) * a.ldx + c0 * KC;
+#pragma unroll
+    for (int cc = 0; cc < KW; ++cc)
+#pragma unroll
+      for (int s = 0; s < SPC; ++s)
+        xa[cc][s] = *reinterpret_cast<const uint4*>(xrow + (cc < kw ? cc : 0) * KC + xcol(s));
+  } else {
+    load4(xr, 0);
+    load4(xn, min(1, ng - 1));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the first tiles' weights ------------------------------------------------------------------------------------
   const long long c0_off = FMT == FMT_NVFP4 ? nv_code_off(c0) : (long long)c0 * unit_bytes(FMT);
   // NVFP4 / FP8 keep two tiles in flight per wave (the 12-wave workgroup leaves 168 VGPRs a lane); INT4's Σx
   // terms leave room for one
@@ -1097,107 +1148,59 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   uint4 u0[KW], s0, u1[KW], s1;
   issue(u0, s0, sb0, 0);
   if (DEPTH > 1) issue(u1, s1, sb1, min(1, ntl - 1));
-
-  // x[token m_row][c0·KC + cc·KC + col(g, s) + (0..7)]: the A operand of step s of chunk cc, col(g, s) =
-  // (KC/4)·g + 8s (NVFP4 / FP8) or 32s + 8g (INT4: the codes' column order in a unit)
-  const bool real = m_row < cnt;
-  auto xcol = [&](int s) { return I4 ? 32 * s + 8 * g : (KC / 4) * g + 8 * s; };
-  uint4 xa[KW][SPC];
-  const uint16_t* xrow = a.x + (long long)(real ? m_row : 0) * a.ldx + c0 * KC;
 #pragma unroll
-  for (int cc = 0; cc < KW; ++cc)
+  for (int cc = 0; cc < KW; ++cc)               // padding tokens: zero operands
 #pragma unroll
     for (int s = 0; s < SPC; ++s)
-      xa[cc][s] = cc < kw ? *reinterpret_cast<const uint4*>(xrow + cc * KC + xcol(s)) : uint4{0u, 0u, 0u, 0u};
-  if (!real) {                                // padding token rows: zero operands (their loads read row 0)
+      if (!F8 || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
+  float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};       // the lane's output tokens are 4g + i: their 2^p
+#pragma unroll 1
+  for (int grp = 0; !F8 && grp < ng; ++grp) {
+    float psr[4];
 #pragma unroll
-    for (int cc = 0; cc < KW; ++cc)
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t vv[4] = {xr[r].x, xr[r].y, xr[r].z, xr[r].w};   // past the slice: its last columns again, unused
+      // the max on the BF16 magnitudes as integers (the same order for finite values)
+      u16x2_t m2 = {0, 0};
 #pragma unroll
-      for (int s = 0; s < SPC; ++s) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
-  }
-
-  if (a.norm_w) {
-    // the norm weights into LDS once; Σx² per token over the row from every wave's slice
-    for (int i = threadIdx.x; i < a.k / 4; i += blockDim.x)
-      reinterpret_cast<float4*>(nws)[i] = reinterpret_cast<const float4*>(a.norm_w)[i];
-    float sq = 0.0f;
+      for (int q = 0; q < 4; ++q) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu));
+      const uint32_t mx = wave_max_u32(max((uint32_t)m2.x, (uint32_t)m2.y));
+      const int pe = mx == 0 ? 0 : (int)(mx >> 7) - 127 - 14;
+      const float inv = __uint_as_float((uint32_t)(127 - pe) << 23);
+      psr[r] = __uint_as_float((uint32_t)(127 + pe) << 23);
+      f16_t h[8];
 #pragma unroll
-    for (int cc = 0; cc < KW; ++cc)
-#pragma unroll
-      for (int s = 0; s < SPC; ++s) {
-        const uint32_t vv[4] = {xa[cc][s].x, xa[cc][s].y, xa[cc][s].z, xa[cc][s].w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q)           // x0² + x1² straight from the BF16 pair: no FP32 copies of the slice
-          sq = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, vv[q]), __builtin_bit_cast(bf16x2, vv[q]), sq, false);
+      for (int q = 0; q < 4; ++q) {
+        h[2 * q] = (f16_t)(bf16_bits_to_f32(vv[q] & 0xFFFFu) * inv);
+        h[2 * q + 1] = (f16_t)(bf16_bits_to_f32(vv[q] >> 16) * inv);
       }
-    sq = add_xor32(add_xor16(active ? sq : 0.0f));    // the four lanes of token m_row
-    if (g == 0) stat[wave * 16 + m_row] = sq;
-    __syncthreads();
-    float t = 0.0f;
-    for (int w = 0; w < S; ++w) t += stat[w * 16 + m_row];
-    const float rr = 1.0f / sqrtf(t / (float)a.k + a.eps);
+      f16x8 o;
 #pragma unroll
-    for (int cc = 0; cc < KW; ++cc)
-#pragma unroll
-      for (int s = 0; s < SPC; ++s) {
-        if (cc >= kw) break;
-        const float* wv = nws + (c0 + cc) * KC + xcol(s);
-        const float4 w0 = *reinterpret_cast<const float4*>(wv), w1 = *reinterpret_cast<const float4*>(wv + 4);
-        const float ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-        uint32_t* vv = reinterpret_cast<uint32_t*>(&xa[cc][s]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float lo = round_bf16((bf16_bits_to_f32(vv[q] & 0xFFFFu) * rr) * ww[2 * q]);
-          const float hi = round_bf16((bf16_bits_to_f32(vv[q] >> 16) * rr) * ww[2 * q + 1]);
-          vv[q] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-        }
-        __builtin_amdgcn_sched_barrier(0);    // one step's weights at a time (the operands already hold 64 VGPRs)
+      for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns,
+      if constexpr (I4) {                                                // 1/16 where the code comes as 16n (exact
+#pragma unroll                                                          // above 2^-10 of a row whose max is 2^14)
+        for (int e = 0; e < 8; ++e)
+          if (int4_high(e)) o[e] *= (f16_t)0.0625f;
       }
-  }
-  // F16 operands: per token, 2^-p brings the slice max into [2^14, 2^15) (exact within 2^28 of the max). The max
-  // is taken on the BF16 magnitudes as integers (same order for finite values), so no FP32 copy of the slice exists.
-  uint32_t mb = 0;
-#pragma unroll
-  for (int cc = 0; cc < KW; ++cc)
-#pragma unroll
-    for (int s = 0; s < SPC; ++s) {
-      const uint32_t vv[4] = {xa[cc][s].x, xa[cc][s].y, xa[cc][s].z, xa[cc][s].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) mb = max(mb, max(vv[q] & 0x7FFFu, (vv[q] >> 16) & 0x7FFFu));
+      *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
     }
-  float mx = bf16_bits_to_f32(mb);
-  mx = max_xor32(max_xor16(mx));
-  const int pe = mx == 0.0f ? 0 : (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127 - 14;
-  const float inv = __uint_as_float((uint32_t)(127 - pe) << 23);
-  const float psc = __uint_as_float((uint32_t)(127 + pe) << 23);
+    wave_lds_sync();
+    if (g == grp) {
 #pragma unroll
-  for (int cc = 0; cc < KW; ++cc)             // in place: xa now holds the F16 operands
-#pragma unroll
-    for (int s = 0; s < SPC; ++s) {
-      uint32_t* vv = reinterpret_cast<uint32_t*>(&xa[cc][s]);
-      if constexpr (I4) {                     // element e of the operand = column int4_perm8(e)
-        uint16_t hv[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) { hv[2 * q] = vv[q] & 0xFFFFu; hv[2 * q + 1] = vv[q] >> 16; }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f16x2 h = {(f16_t)(bf16_bits_to_f32(hv[int4_perm8(2 * q)]) * inv),
-                           (f16_t)(bf16_bits_to_f32(hv[int4_perm8(2 * q + 1)]) * inv)};
-          vv[q] = __builtin_bit_cast(uint32_t, h);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f16x2 h = {(f16_t)(bf16_bits_to_f32(vv[q] & 0xFFFFu) * inv), (f16_t)(bf16_bits_to_f32(vv[q] >> 16) * inv)};
-          vv[q] = __builtin_bit_cast(uint32_t, h);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);      // one operand at a time: no FP32 copies of the whole slice
+      for (int r = 0; r < 4; ++r) ps[r] = psr[r];
     }
-  // the output rows of lane l are tokens 4g + i: their scales from the lanes that hold those tokens' A rows
-  float ps[4];
+    if ((m_row >> 2) == grp && m_row < cnt) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) ps[i] = __shfl(psc, 4 * g + i, 64);
+      for (int cc = 0; cc < KW; ++cc)
+#pragma unroll
+        for (int s = 0; s < SPC; ++s)
+          xa[cc][s] = *reinterpret_cast<const uint4*>(stage + (m_row & 3) * ROWM_SLD + 2 * (cc * KC + xcol(s)));
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) xr[r] = xn[r];
+    if (grp + 2 < ng) load4(xn, grp + 2);
+  }
   // INT4: Σx (prescaled F16) per 64-column group — steps {0, 1} and {2, 3} of each chunk — per token (the sum over
   // its four k-group lanes), kept in the wave's LDS rows: tile_mma reads those of its output tokens 4g + i
   float* sxw = sxl + wave * KW * 2 * 16;
@@ -1211,10 +1214,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         for (int s = 2 * gp; s < 2 * gp + 2; ++s) {
           const f16x8 h = __builtin_bit_cast(f16x8, xa[cc][s]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) sx += (float)h[e];
+          for (int e = 0; e < 8; ++e) sx += (float)h[e] * (int4_high(e) ? 16.0f : 1.0f);
         }
         sx = add_xor32(add_xor16(cc < kw ? sx : 0.0f));
-        if (g == 0) sxw[(cc * 2 + gp) * 16 + m_row] = sx;
+        if (g == 0) sxw[(cc * 2 + gp) * 16 + m_row] = sx * 0x1p-24f;     // in the units of the codes' dot products
       }
     wave_lds_sync();
   }
@@ -1232,19 +1235,18 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
                                  : __builtin_amdgcn_cvt_pk_f32_fp8((int)word, false);
         const uint32_t b0 = __float_as_uint(f.x), b1 = __float_as_uint(f.y);
         const float e0 = __uint_as_float(b0 & 0x7F800000u), e1 = __uint_as_float(b1 & 0x7F800000u);
-        const f16_t m0 = (f16_t)nv_mant(b0);
-        const f16_t m1 = (f16_t)nv_mant(b1);
+        const f16x2 mm = {(f16_t)nv_mant_f16(b0), (f16_t)nv_mant_f16(b1)};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-          const f16x8 bv = nvfp4_decode8(dw[s], s < 2 ? e0 : e1, s < 2 ? m0 : m1);
+          const f16x8 bv = nvfp4_decode8(dw[s], s < 2 ? e0 : e1, s < 2 ? mm.x : mm.y);
           acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][s]), bv, acc, 0, 0, 0);
         }
       } else if constexpr (I4) {                // the two 64-column groups, each scaled and offset on its own
         f32x4 da = {0.f, 0.f, 0.f, 0.f}, db = {0.f, 0.f, 0.f, 0.f};
-        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][0]), int4_decode8(dw[0]), da, 0, 0, 0);
-        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][1]), int4_decode8(dw[1]), da, 0, 0, 0);
-        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][2]), int4_decode8(dw[2]), db, 0, 0, 0);
-        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][3]), int4_decode8(dw[3]), db, 0, 0, 0);
+        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][0]), int4_decode8_denormal(dw[0]), da, 0, 0, 0);
+        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][1]), int4_decode8_denormal(dw[1]), da, 0, 0, 0);
+        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][2]), int4_decode8_denormal(dw[2]), db, 0, 0, 0);
+        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][3]), int4_decode8_denormal(dw[3]), db, 0, 0, 0);
         const uint2 sb = sbs[cc];
         const float sca = bf16_bits_to_f32(sb.x & 0xFFFFu), bia = bf16_bits_to_f32(sb.x >> 16);
         const float scb = bf16_bits_to_f32(sb.y & 0xFFFFu), bib = bf16_bits_to_f32(sb.y >> 16);
@@ -1258,15 +1260,16 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       } else {                                  // FP8: the lane's 16 codes, 8 per step
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          const f16x8 bv = fp8_decode8(dw[2 * s], dw[2 * s + 1]);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][s]), bv, acc, 0, 0, 0);
+          const bf16x8 bv = fp8_decode8_bf16(dw[2 * s], dw[2 * s + 1]);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[cc][s]), bv, acc, 0, 0, 0);
         }
       }
       __builtin_amdgcn_sched_barrier(0);      // decode chunk by chunk: keeps the decoded operands' registers few
     }
-    float* rp = red + ((jt * S + wave) * 16) * 16;
+    float* rp = red + wave * a.row_ld + jt * 256;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rp[(4 * g + i) * 16 + m_row] = active ? acc[i] * ps[i] : 0.0f;
+    for (int i = 0; i < 4; ++i)
+      rp[(4 * g + i) * 16 + m_row] = active ? (F8 ? acc[i] : acc[i] * (I4 ? ps[i] * 0x1p24f : ps[i])) : 0.0f;
   };
   if constexpr (DEPTH == 1) {
     for (int j = 0; j < ntl; ++j) {
@@ -1279,15 +1282,6 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     // flight there is waited for where its registers are reused (a round trip on every wave's way out), so the
     // tail's call sites are spelled out.
     int j = 0;
-    if constexpr (FMT == FMT_FP8) {             // the longer FP8 decode: the spelled-out tail spills (40 B / lane)
-      for (; j + 1 < ntl; j += 2) {
-        tile_mma(u0, s0, sb0, j);
-        issue(u0, s0, sb0, min(j + 2, ntl - 1));
-        tile_mma(u1, s1, sb1, j + 1);
-        issue(u1, s1, sb1, min(j + 3, ntl - 1));
-      }
-      if (j < ntl) tile_mma(u0, s0, sb0, j);
-    } else {
     for (; j + 3 < ntl; j += 2) {
       tile_mma(u0, s0, sb0, j);
       issue(u0, s0, sb0, j + 2);
@@ -1305,23 +1299,33 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     } else {
       tile_mma(u0, s0, sb0, j);
     }
-    }
   }
 
-  // ---- per (tile, token): the K slices in the gemv_row order, then the epilogue --------------------------------
+  // ---- per (tile, token, row): the K slices in the gemv_row order, then the epilogue. A lane per value — a wave takes
+  // 4 tokens × 16 rows of one tile a step — so its at most 12 LDS reads, issued together, are the whole chain, and the
+  // row scales of its steps come before the barrier. (A wave per (tile, token), 16 of its lanes storing, with the row
+  // scale loaded in the loop, took 5 us more on the 27B gate|up at M = 16; unrolled over a wave's steps, the code's first
+  // fetch cost what the overlap gained, so the loop stays rolled) -----------------------------------------------------
+  const int tq = (cnt + 3) >> 2, steps = ntl * tq, inv_tq = 65536 / tq + 1;      // st / tq = st·inv_tq >> 16 (tq <= 4)
+  auto load_rs = [&](int st) {
+    return a.row_scale != nullptr && a.ks == 1
+               ? a.row_scale[tile_of((min(st, steps - 1) * inv_tq) >> 16) * 16 + m_row] : 1.0f;
+  };
+  float rs = load_rs(wave);
   __syncthreads();
-  for (int pi = wave; pi < ntl * cnt; pi += S) {
-    const int jt = pi / cnt, t = pi - jt * cnt;
-    const int tile = tile_of(jt);
-    float v = slice_sum(red + (jt * S * 16 + t) * 16, 16 * 16, S, lane);
-    const int row = tile * 16 + m_row;
+#pragma unroll 1
+  for (int st = wave; st < steps; st += S) {
+    const int jt = (st * inv_tq) >> 16, t = 4 * (st - jt * tq) + g, tile = tile_of(jt), row = tile * 16 + m_row;
+    const float rs_st = rs;
+    rs = load_rs(st + S);
+    float v = slice_sum12(red + jt * 256 + t * 16 + m_row, a.row_ld, S);
     if (a.ks > 1) {
-      if (g == 0) a.part[((long long)split * a.m + t) * a.n_tiles * 16 + row] = v;
+      if (t < cnt) a.part[((long long)split * a.m + t) * a.n_tiles * 16 + row] = v;
       continue;
     }
-    v *= a.row_scale != nullptr ? a.row_scale[row] : 1.0f;
+    v *= rs_st;
     const float up = __shfl_down(v, 8, 16);
-    if (g == 0) emit(a, a.epilogue, nullptr, cnt, tile, true, m_row, t, v, up);
+    emit(a, a.epilogue, nullptr, cnt, tile, true, m_row, t, v, up);
   }
 }
 
@@ -2218,42 +2222,40 @@ int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
 
 Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   Plan best{};
-  if ((d->format != FMT_NVFP4 && d->format != FMT_FP8 && d->format != FMT_INT4) || d->groups || d->gnorm_w ||
+  if ((d->format != FMT_NVFP4 && d->format != FMT_FP8 && d->format != FMT_INT4) || d->groups || d->gnorm_w || d->norm_w ||
       d->m < 3 || d->m > 16 ||
       (d->format == FMT_NVFP4 && chunks % 4))     // NVFP4 slices start on half scale groups
     return best;
   const int kw = 512 / chunk_cols(d->format);    // chunks per wave (512 columns)
   int ks = (chunks + 12 * kw - 1) / (12 * kw);   // at most 12 waves: the kernel's VGPR budget is 3 waves per SIMD
-  if (d->norm_w && ks > 1) return best;          // the fused norm needs the whole row in one workgroup
   int force_ks = 0, force_rt = 0;
   if (const char* env = getenv("MI_GEMV_ROWM")) {                                // tuning sweeps
     const char* ke = getenv("MI_GEMV_ROWM_K");                                   // only launches of this K
     if (!ke || atoi(ke) == d->k) sscanf(env, "%d,%d", &force_ks, &force_rt);
   }
   if (force_ks) ks = force_ks;
-  // one split whose tiles' waves fill under three quarters of the chip's wave slots (12 per CU at this kernel's
-  // VGPR budget): three K splits, so the tiles spread over every CU (27B attention o_proj at M = 8, 320 tiles of 6
-  // waves: 14.0 → 11.6 µs with the reduction launch; out_proj's 12 waves per tile measured best unsplit)
-  if (!force_ks && ks == 1 && !d->norm_w && (long long)n_tiles * ((chunks + kw - 1) / kw) * 4 < 3LL * cu_count() * 12) {
-    const int kc3 = ((chunks + 2) / 3 + 7) / 8 * 8;
-    if (2 * kc3 < chunks) ks = 3;                // three non-empty splits on scale-group boundaries
-  }
   int kc = (chunks + ks - 1) / ks;
   if (ks > 1) kc = (kc + 7) / 8 * 8;             // splits on scale-group boundaries (whole waves for FP8)
   if (kc > 12 * kw || (ks > 1 && (ks - 1) * kc >= chunks)) return best;
   const int S = (kc + kw - 1) / kw;
-  const size_t fixed = (d->norm_w ? (size_t)d->k * 4 : 0) + (size_t)S * 16 * 4 +
-                       (d->format == FMT_INT4 ? (size_t)S * (512 / chunk_cols(FMT_INT4)) * 2 * 16 * 4 : 0);
-  const size_t per_tile = (size_t)S * 16 * 16 * 4;
-  const int per_cu = rowm_blocks_per_cu(d->format, 64 * S, fixed + 4 * per_tile);
-  const long long slots = std::max<long long>(1, (long long)cu_count() * std::max(per_cu, 1) / ks);
-  // every resident slot takes tiles (strided), so no CU idles for the rounding of tiles per workgroup
+  const size_t fixed = d->format == FMT_INT4 ? (size_t)S * (512 / chunk_cols(FMT_INT4)) * 2 * 16 * 4 : 0;
+  // a wave's LDS region: its activation stage (4 rows), then a 1 KiB partial per tile
+  auto region = [](int rt) { return std::max<size_t>(4 * ROWM_SLD, (size_t)rt * 1024); };
+  const int per_cu = rowm_blocks_per_cu(d->format, 64 * S, fixed + S * region(4));
+  // Workgroups per CU: as many as make six waves, at least one. The activations are converted once per workgroup, on
+  // every CU the same work for each resident workgroup, so fewer workgroups over more tiles win as long as a CU has
+  // about four waves' loads in flight (one workgroup of 6 waves a CU over 6 tiles instead of two over 3, N = 24576,
+  // K = 3072, M = 8: 16.3 → 12.6 us; N = 5120, K = 3072: 10.6 → 7.5 us, where three K splits and their reduction launch
+  // took 9.9; two waves a workgroup need three: 10.4 → 8.8 us). K is split only where it does not fit 12 waves.
+  const int per_cu_want = std::min(std::max(per_cu, 1), std::max(1, 6 / S));
+  const long long slots = std::max<long long>(1, (long long)cu_count() * per_cu_want / ks);
+  // every slot takes tiles (strided), so no CU idles for the rounding of tiles per workgroup
   int G = (int)std::min<long long>(n_tiles, slots);
   if (force_rt) G = (n_tiles + force_rt - 1) / force_rt;
   const int rt = (n_tiles + G - 1) / G;
-  const size_t lds = fixed + (size_t)rt * per_tile;
+  const size_t lds = fixed + S * region(rt);
   if (lds > kMaxLds) return best;
-  best.kernel = 3; best.S = S; best.kw = kc; best.ks = ks; best.rt = rt; best.G = G;
+  best.kernel = 3; best.row_ld = (int)(region(rt) / 4); best.S = S; best.kw = kc; best.ks = ks; best.rt = rt; best.G = G;
   best.tb = rt; best.lds_rows = 16; best.lds_bytes = lds;
   return best;
 }
@@ -2273,9 +2275,8 @@ size_t fold_counter_bytes(int) { return kFoldCounterBytes; }
 // behind a workgroup barrier. Measured on the 27B shapes at M = 8, bit-identical: gate|up 33.0 → 30.5 µs, in_proj
 // 24.7 → 22.0 µs (the extra launch ≈ 2.9 µs). At M <= 2 gemv_row's fused norm costs less than a launch.
 bool wants_prenorm(const mi_gemv_desc* d) {
-  static const bool off = getenv("MI_GEMV_PRENORM") && getenv("MI_GEMV_PRENORM")[0] == '0';   // A/B comparisons
   const int rows = d->groups ? std::min(16, d->m) : d->m;
-  return !off && d->norm_w && rows > 2 && !(d->groups && d->x_per_slot) && !d->route_logits && d->k % 8 == 0;
+  return d->norm_w && rows > 2 && !(d->groups && d->x_per_slot) && !d->route_logits && d->k % 8 == 0;
 }
 
 Plan make_plan(const mi_gemv_desc* d) {
@@ -2355,10 +2356,7 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
       return p;
     }
   }
-  // INT4 at M >= 3 runs on gemv_tk unless gemv_rowm is pinned: measured on the 27B gate|up shape at M = 8,
-  // gemv_rowm takes 37.4 µs against gemv_tk's 35.5 (its per-group scale / bias work is VALU time the NVFP4 decode
-  // does not have), although gemv_tk moves 11 MB of split partials more
-  if (rows > 2 && !pin_tk && (fmt != FMT_INT4 || pin_rowm)) {
+  if (rows > 2 && !pin_tk) {
     const Plan p = plan_rowm(d, chunks, n_tiles);
     if (p.kernel) return p;
   }

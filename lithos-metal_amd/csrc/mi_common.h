@@ -81,6 +81,18 @@ __device__ __forceinline__ float max16(float v) {
   return v;
 }
 
+// the largest of the wave's integers, in every lane
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppXor2, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppHalfMirror, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppMirror, 0xF, 0xF, true));
+  const auto r = __builtin_amdgcn_permlane16_swap((int)v, (int)v, false, false);
+  v = max((uint32_t)r[0], (uint32_t)r[1]);
+  const auto q = __builtin_amdgcn_permlane32_swap((int)v, (int)v, false, false);
+  return max((uint32_t)q[0], (uint32_t)q[1]);
+}
+
 // v(l) + v(l ^ 16) and v(l) + v(l ^ 32): a swap leaves each lane holding its own value in one half of the pair and
 // its partner's in the other, so the pair's sum (max) is the same in both lanes
 __device__ __forceinline__ float add_xor16(float v) {

@@ -40,6 +40,9 @@ __device__ __forceinline__ float nv_mant(uint32_t u) {
   return __uint_as_float((u & 0x7F800000u) ? ((u & 0x807FFFFFu) | 0x3F800000u) : (u & 0x80000000u));
 }
 
+// the same where the codes become F16: a zero scale's 2^-127 codes are then 0 already
+__device__ __forceinline__ float nv_mant_f16(uint32_t u) { return __uint_as_float((u & 0x807FFFFFu) | 0x3F800000u); }
+
 // byte j of dw (two E2M1 codes, low nibble first) → BF16 pair × 2^E (exact); j is a compile-time constant after
 // unrolling, as the instruction's byte select requires
 __device__ __forceinline__ bf16x2 cvt_fp4x2_bf16(uint32_t dw, float e, int j) {
@@ -102,6 +105,17 @@ __device__ __forceinline__ float slice_sum_lane(const float* red, int stride, in
     p[q] = 0.0f;
     for (int w = q; w < S; w += 4) p[q] += red[w * stride + r];
   }
+  return (p[0] + p[1]) + (p[2] + p[3]);
+}
+
+// slice_sum_lane for at most 12 slices, every read issued before the first is used (a slice past the last re-reads the
+// last and adds +0, which leaves a sum that began at +0 as it is)
+__device__ __forceinline__ float slice_sum12(const float* red, int stride, int S) {
+  float x[12], p[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int w = 0; w < 12; ++w) x[w] = red[min(w, S - 1) * stride];
+#pragma unroll
+  for (int w = 0; w < 12; ++w) p[w & 3] += w < S ? x[w] : 0.0f;
   return (p[0] + p[1]) + (p[2] + p[3]);
 }
 

@@ -272,6 +272,27 @@ def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch
     assert chk.ok_rounded() and chk.within, (mtok, n, k, plan, epi, chk)
 
 
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3"])
+@pytest.mark.parametrize("mtok", [3, 4, 5, 8, 9, 13, 16])
+@pytest.mark.parametrize("n,k", [(24, 128), (4117, 640), (40, 6656)])
+def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
+    """Every remainder of the four rows staged at a time, a slice of one chunk, one more tile than workgroups, two K
+    splits; a row of zeros, one scaled by 2^60 and one by 2^-60 (each row's own power-of-two prescale): every row
+    inside the leaf gate of its own values."""
+    m = _matrix(fmt, n, k, rng)
+    x = rbf(rng.standard_normal((mtok, k)).astype(np.float32))
+    x[0] = 0.0
+    x[1] *= 2.0 ** 60
+    x[mtok - 1] *= 2.0 ** -60
+    got = _run(torch_gpu, m, x)
+    ref = ON.matmul_acc(x, _dequant(m))
+    assert not got[0].any()
+    for i in range(1, mtok):
+        e = (0, 60)[i == 1] or (0, -60)[i == mtok - 1]
+        chk = check_against_oracle(got[i: i + 1] * np.float32(2.0 ** -e), ref[i: i + 1] * np.float32(2.0 ** -e))
+        assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
+
+
 def test_fp8_dequant_every_code(torch_gpu):
     """Every finite E4M3 code (signed zero, subnormals, ±448) decodes bit-exactly; the tensor scale multiplies once."""
     from monolith_mi355 import kernels
