@@ -1787,18 +1787,14 @@ __global__ __launch_bounds__(256) void gemv_tk_reduce(Args a) {
 
 // The split-K reduction of a dense GEMV with BF16 output (epilogue none or residual) and the next RMSNorm of its
 // output in one launch: y as gemv_tk_reduce writes it (splits added in order, row scale, residual, one BF16
-// rounding), then x_next as norm_apply computes it over y. One workgroup of RN_NT threads per token, a thread per
-// 8-column vector: all its loads (partials of every split at a clamped index, residual, row scales, norm weights)
-// issued up front, so the launch waits one memory round trip; y goes to LDS, where the first RN_SUM threads take
-// Σ y² exactly as norm_apply's threads do (vectors tid, tid + RN_SUM, … in order, fma, then the waves in order) —
-// the same statistic, bit for bit — and every thread normalizes its vector (n <= 8·RN_NT, at most RN_KS splits).
+// rounding), then x_next as norm_apply computes it over y. One workgroup per token, a thread per 8-column vector: all
+// its loads (partials of every split at a clamped index, residual, row scales, norm weights) issued up front, so the
+// launch waits one memory round trip; a wave's vectors are one slice of the statistic, as in norm_apply — the same
+// bits — and every thread normalizes its vector (n <= 8·RN_NT, at most RN_KS splits).
 constexpr int RN_NT = 1024;
-constexpr int RN_SUM = 256;     // norm_apply's workgroup: its per-thread vectors fix the order of Σ
 constexpr int RN_KS = 4;
 __global__ __launch_bounds__(RN_NT) void gemv_reduce_norm(Args a) {
-  __shared__ __attribute__((aligned(16))) uint4 ys[RN_NT];
-  __shared__ float red[RN_SUM / 64];
-  __shared__ float rsh;
+  __shared__ float red[RN_NT / 64];
   const int t = blockIdx.x, tid = threadIdx.x;
   const int n_pad = a.n_tiles * 16, nv = a.n / 8;
   const bool resid = a.epilogue == MI_EPI_RESIDUAL;
@@ -1838,44 +1834,15 @@ __global__ __launch_bounds__(RN_NT) void gemv_reduce_norm(Args a) {
     }
     yb[i] = f32_to_bf16_bits(lo) | ((uint32_t)f32_to_bf16_bits(hi) << 16);
   }
-  const uint4 y4{yb[0], yb[1], yb[2], yb[3]};
-  if (tid < nv) {
-    *reinterpret_cast<uint4*>(a.y + (long long)t * a.ldy + 8 * tid) = y4;
-    ys[tid] = y4;
-  }
+  if (tid < nv) *reinterpret_cast<uint4*>(a.y + (long long)t * a.ldy + 8 * tid) = uint4{yb[0], yb[1], yb[2], yb[3]};
+  const float sv = vec_sumsq(yb), s = wave_sum(tid < nv ? sv : 0.0f);
+  if ((tid & 63) == 0) red[tid >> 6] = s;
   lds_barrier();
-  if (tid < RN_SUM) {
-    float s = 0.0f;
-    for (int jj = tid; jj < nv; jj += RN_SUM) {
-      const uint4 q = ys[jj];
-      const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float lo = bf16_bits_to_f32(qw[i] & 0xFFFFu), hi = bf16_bits_to_f32(qw[i] >> 16);
-        s = fmaf(lo, lo, s);
-        s = fmaf(hi, hi, s);
-      }
-    }
-    s = wave_sum(s);
-    if ((tid & 63) == 0) red[tid >> 6] = s;
-  }
-  lds_barrier();
-  if (tid == 0) {
-    float ssq = 0.0f;
-#pragma unroll
-    for (int w = 0; w < RN_SUM / 64; ++w) ssq += red[w];
-    rsh = 1.0f / sqrtf(ssq / (float)a.n + a.nn_eps);
-  }
-  lds_barrier();
-  const float r = rsh;
-  const float w8[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+  float ssq = 0.0f;
+  for (int i = 0; i < (a.n + STAT_SLICE - 1) / STAT_SLICE; ++i) ssq += red[i];
+  const float r = 1.0f / sqrtf(ssq / (float)a.n + a.nn_eps);
   uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float lo = round_bf16((bf16_bits_to_f32(yb[i] & 0xFFFFu) * r) * w8[2 * i]);
-    const float hi = round_bf16((bf16_bits_to_f32(yb[i] >> 16) * r) * w8[2 * i + 1]);
-    o[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-  }
+  norm_vec(yb, r, w0, w1, o);
   if (tid < nv) *reinterpret_cast<uint4*>(a.nn_x + (long long)t * a.ld_nn_x + 8 * tid) = uint4{o[0], o[1], o[2], o[3]};
 }
 
@@ -2273,7 +2240,9 @@ size_t fold_counter_bytes(int) { return kFoldCounterBytes; }
 // GEMV reads the normalized rows: inside gemv_rowm / gemv_tk every workgroup would normalize the whole [M, K] input
 // again (per element: two multiplies and a BF16 rounding, on operand lanes of which half are padding rows at M = 8)
 // behind a workgroup barrier. Measured on the 27B shapes at M = 8, bit-identical: gate|up 33.0 → 30.5 µs, in_proj
-// 24.7 → 22.0 µs (the extra launch ≈ 2.9 µs). At M <= 2 gemv_row's fused norm costs less than a launch.
+// 24.7 → 22.0 µs (the extra launch ≈ 2.9 µs). Inside gemv_rowm's staging of four rows at a time (statistic through LDS,
+// one barrier a group) it still measured 2 to 4 us a group more than the launch: gate|up at M = 3 / 8 / 16 23.5 / 23.8 /
+// 27.7 us with the launch, 27.0 / 31.4 / 39.4 fused. At M <= 2 gemv_row's fused norm costs less than a launch.
 bool wants_prenorm(const mi_gemv_desc* d) {
   const int rows = d->groups ? std::min(16, d->m) : d->m;
   return d->norm_w && rows > 2 && !(d->groups && d->x_per_slot) && !d->route_logits && d->k % 8 == 0;
@@ -2401,7 +2370,7 @@ void launch_row_k(const Args& a, const Plan& p, dim3 g, hipStream_t s) {
 // the split-K reduction launch: with the next norm (a.nn_w), gemv_reduce_norm; else gemv_tk_reduce
 void launch_reduce(const Args& a, hipStream_t s) {
   if (a.nn_w) {
-    hipLaunchKernelGGL(gemv_reduce_norm, dim3(a.m), dim3(RN_NT), 0, s, a);
+    hipLaunchKernelGGL(gemv_reduce_norm, dim3(a.m), dim3((a.n / 8 + 63) / 64 * 64), 0, s, a);
     return;
   }
   const bool silu = a.epilogue == MI_EPI_SILU_MUL || a.epilogue == MI_EPI_SILU_MUL_ROUNDED;

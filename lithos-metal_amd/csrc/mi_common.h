@@ -117,3 +117,30 @@ __device__ __forceinline__ float quad16_sum(float v) { return add_xor32(add_xor1
 
 __device__ __forceinline__ float wave_sum(float v) { return quad16_sum(sum16(v)); }
 __device__ __forceinline__ float wave_max(float v) { return max_xor32(max_xor16(max16(v))); }
+
+// ---- the RMSNorm statistic Σ x² of a BF16 row, in one order wherever it is taken (norm_apply, rmsnorm_stat, the
+// reductions and the combine that write the next layer's normalized rows, gemv_rowm's fused norm): the 8-column vector
+// of a lane by fma in column order from 0, the 64 vectors of a 512-column slice by wave_sum, the slices in order. A wave
+// then holds a slice wherever its kernel has it, and the slices meet in LDS.
+constexpr int STAT_SLICE = 512;
+__device__ __forceinline__ float vec_sumsq(const uint32_t (&v)[4]) {
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float lo = bf16_bits_to_f32(v[i] & 0xFFFFu), hi = bf16_bits_to_f32(v[i] >> 16);
+    s = fmaf(lo, lo, s);
+    s = fmaf(hi, hi, s);
+  }
+  return s;
+}
+
+// 8 values of a normalized row: bf16((x·r)·w)
+__device__ __forceinline__ void norm_vec(const uint32_t (&v)[4], float r, const float4 w0, const float4 w1, uint32_t (&o)[4]) {
+  const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float lo = round_bf16((bf16_bits_to_f32(v[i] & 0xFFFFu) * r) * w[2 * i]);
+    const float hi = round_bf16((bf16_bits_to_f32(v[i] >> 16) * r) * w[2 * i + 1]);
+    o[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
+  }
+}

@@ -188,58 +188,26 @@ __global__ __launch_bounds__(256) void moe_combine(CombineArgs a) {
   *reinterpret_cast<uint4*>(a.out + (long long)t * a.ldo + c) = combine_vec(a, t, c);
 }
 
-// The combine with the next RMSNorm of its output (the next layer's normalized input): one workgroup of 1024 per
-// token, a thread per 8-column vector; the output goes to LDS, where the first 256 threads take Σ out² as
-// norm_apply's threads do (vectors tid, tid + 256, … in order, fma, then the waves in order) — the same statistic,
-// bit for bit — and every thread normalizes its vector: x = bf16((out·r)·w). hidden <= 8192.
+// The combine with the next RMSNorm of its output (the next layer's normalized input): one workgroup per token, a thread
+// per 8-column vector; a wave's vectors are one slice of the statistic, as in norm_apply — the same bits — and every
+// thread normalizes its vector: x = bf16((out·r)·w). hidden <= 8192.
 constexpr int CN_NT = 1024;
-constexpr int CN_SUM = 256;
 __global__ __launch_bounds__(CN_NT) void moe_combine_norm(CombineArgs a) {
-  __shared__ __attribute__((aligned(16))) uint4 ys[CN_NT];
-  __shared__ float red[CN_SUM / 64];
-  __shared__ float rsh;
+  __shared__ float red[CN_NT / 64];
   const int t = blockIdx.x, tid = threadIdx.x, nv = a.hidden / 8;
   const int c = 8 * min(tid, nv - 1);
   const float4 w0 = *reinterpret_cast<const float4*>(a.nn_w + c), w1 = *reinterpret_cast<const float4*>(a.nn_w + c + 4);
   const uint4 o = combine_vec(a, t, c);
-  if (tid < nv) {
-    *reinterpret_cast<uint4*>(a.out + (long long)t * a.ldo + 8 * tid) = o;
-    ys[tid] = o;
-  }
-  lds_barrier();
-  if (tid < CN_SUM) {
-    float s = 0.0f;
-    for (int jj = tid; jj < nv; jj += CN_SUM) {
-      const uint4 q = ys[jj];
-      const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float lo = bf16_bits_to_f32(qw[i] & 0xFFFFu), hi = bf16_bits_to_f32(qw[i] >> 16);
-        s = fmaf(lo, lo, s);
-        s = fmaf(hi, hi, s);
-      }
-    }
-    s = wave_sum(s);
-    if ((tid & 63) == 0) red[tid >> 6] = s;
-  }
-  lds_barrier();
-  if (tid == 0) {
-    float ssq = 0.0f;
-#pragma unroll
-    for (int w = 0; w < CN_SUM / 64; ++w) ssq += red[w];
-    rsh = 1.0f / sqrtf(ssq / (float)a.hidden + a.nn_eps);
-  }
-  lds_barrier();
-  const float r = rsh;
+  if (tid < nv) *reinterpret_cast<uint4*>(a.out + (long long)t * a.ldo + 8 * tid) = o;
   const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
-  const float w8[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+  const float sv = vec_sumsq(ow), s = wave_sum(tid < nv ? sv : 0.0f);
+  if ((tid & 63) == 0) red[tid >> 6] = s;
+  lds_barrier();
+  float ssq = 0.0f;
+  for (int i = 0; i < (a.hidden + STAT_SLICE - 1) / STAT_SLICE; ++i) ssq += red[i];
+  const float r = 1.0f / sqrtf(ssq / (float)a.hidden + a.nn_eps);
   uint32_t xo[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float lo = round_bf16((bf16_bits_to_f32(ow[i] & 0xFFFFu) * r) * w8[2 * i]);
-    const float hi = round_bf16((bf16_bits_to_f32(ow[i] >> 16) * r) * w8[2 * i + 1]);
-    xo[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-  }
+  norm_vec(ow, r, w0, w1, xo);
   if (tid < nv) *reinterpret_cast<uint4*>(a.nn_x + (long long)t * a.ld_nn_x + 8 * tid) = uint4{xo[0], xo[1], xo[2], xo[3]};
 }
 
@@ -297,7 +265,7 @@ extern "C" int mi_moe_combine(const mi_moe_combine_desc* d, void* stream) {
       a.nn_x = d->next_x;
       a.ld_nn_x = d->ld_next_x;
       a.nn_eps = d->next_eps;
-      hipLaunchKernelGGL(moe_combine_norm, dim3(d->t), dim3(CN_NT), 0, static_cast<hipStream_t>(stream), a);
+      hipLaunchKernelGGL(moe_combine_norm, dim3(d->t), dim3((d->hidden / 8 + 63) / 64 * 64), 0, static_cast<hipStream_t>(stream), a);
       MI_TRY_HIP(hipGetLastError(), "moe_combine_norm launch");
       return MI_OK;
     }
