@@ -2190,7 +2190,7 @@ int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
 Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   Plan best{};
   if ((d->format != FMT_NVFP4 && d->format != FMT_FP8 && d->format != FMT_INT4) || d->groups || d->gnorm_w || d->norm_w ||
-      d->m < 3 || d->m > 16 ||
+      d->m < 2 || d->m > 16 ||
       (d->format == FMT_NVFP4 && chunks % 4))     // NVFP4 slices start on half scale groups
     return best;
   const int kw = 512 / chunk_cols(d->format);    // chunks per wave (512 columns)
@@ -2248,7 +2248,28 @@ bool wants_prenorm(const mi_gemv_desc* d) {
   return d->norm_w && rows > 2 && !(d->groups && d->x_per_slot) && !d->route_logits && d->k % 8 == 0;
 }
 
-Plan make_plan(const mi_gemv_desc* d) {
+// Two tokens over a large weight stream run on gemv_rowm: gemv_row's dot products for two tokens (VALU) fall behind the
+// stream, the matrix cores take any M at the price of one, and the norm's launch costs less than normalizing two rows
+// in every workgroup. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 42.9 → 23.3 us, without 29.0 →
+// 20.7, in_proj with the norm 23.4 → 15.5, down 17.0 → 15.0, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
+// MB, norm) 11.5 → 10.8; below that gemv_row wins: N = 12288, K = 2048 (14.2 MB, norm) 7.9 against 8.1, FP8 4096 x 4096
+// (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4.
+constexpr size_t kRowmTwoBytes = 20u << 20;
+bool rowm_at_two(const mi_gemv_desc* d) {
+  return d->m == 2 && !d->groups && !d->gnorm_w && !d->conv_w && d->format != FMT_BF16 &&
+         (size_t)((d->n + 15) / 16) * (size_t)tile_bytes(d->format, d->k / chunk_cols(d->format)) >= kRowmTwoBytes &&
+         !getenv("MI_GEMV_KERNEL") && !getenv("MI_GEMV_ROW");
+}
+
+// two: whether two tokens may take gemv_rowm, which needs scratch where gemv_row does not
+Plan make_plan(const mi_gemv_desc* d, bool two = true) {
+  if (two && rowm_at_two(d)) {
+    mi_gemv_desc plain = *d;
+    plain.norm_w = nullptr;
+    Plan p = plan_rowm(&plain, d->k / chunk_cols(d->format), (d->n + 15) / 16);
+    p.prenorm = p.kernel != 0 && d->norm_w;
+    if (p.kernel) return p;
+  }
   if (d->conv_w) {                              // the conv epilogue lives in gemv_row: one tile per workgroup
     Plan p = make_plan_fused(d);
     if (p.kernel == 1 && p.rt > 1) {
@@ -2442,8 +2463,20 @@ namespace {
 // device-resident array), or null: the caller's workspace, else the library's scratch.
 int gemv_impl(const mi_gemv_desc* d, void* stream, void* fixed_ws, size_t fixed_bytes, const char* name) {
   if (int rc = check_desc(d)) return rc;
-  const Plan p = make_plan(d);
+  Plan p = make_plan(d);
   MI_REQUIRE(p.kernel, "%s: no launch plan fits (k=%d, m=%d)", name, d->k, d->m);
+  // two tokens on gemv_rowm without the scratch it needs (a workspace sized for less, a stream captured before its first
+  // eager call): gemv_row
+  void* unused = nullptr;
+  if (p.kernel == 3 && d->m == 2) {
+    if (const size_t need = workspace_need(d, p)) {
+      const bool ok = fixed_ws ? need <= fixed_bytes
+                      : d->workspace ? d->workspace_bytes >= need
+                                     : mi_library_scratch(MI_SCRATCH_GEMV, need, static_cast<hipStream_t>(stream), &unused) == MI_OK;
+      if (!ok) p = make_plan(d, false);
+      MI_REQUIRE(p.kernel, "%s: no launch plan fits (k=%d, m=%d)", name, d->k, d->m);
+    }
+  }
   MI_REQUIRE(!d->route_logits || (p.kernel == 1 && p.ks == 1), "%s: routing in the launch runs on gemv_row", name);
   Args a{};
   a.w = static_cast<const uint8_t*>(d->w);

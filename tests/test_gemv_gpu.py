@@ -293,6 +293,39 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
         assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
 
 
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3"])
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("norm", [False, True])
+def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
+    """Two tokens on either side of the weight bytes where gemv_rowm takes over (20 MiB): the plan, the rows against the
+    oracle's float64 product, and a workspace too small for gemv_rowm's scratch (then gemv_row, the same gate)."""
+    import ctypes as C
+    from monolith_mi355 import kernels
+    from monolith_mi355.runtime import hip
+    torch = torch_gpu
+    k = 1024
+    per_row = {"nvfp4": 576, "int4_affine": 576, "fp8_e4m3": 1024}[fmt]
+    n = ((20 << 20) // (per_row * 16) + (1 if big else -1)) * 16
+    block = _matrix(fmt, 512, k, rng)                       # 512 random rows down the matrix
+    rep = -(-n // 512)
+    m = {kk: (np.tile(v, (rep, 1))[:n].copy() if isinstance(v, np.ndarray) and v.ndim == 2 else v) for kk, v in block.items()}
+    x = rbf(rng.standard_normal((2, k)).astype(np.float32))
+    nw = (1.0 + rng.standard_normal(k) * 0.1).astype(np.float32)
+    w, xd = _upload(torch, m), to_dev_bf16(torch, x)
+    kw = dict(norm_w=torch.from_numpy(nw).cuda(), eps=1e-6) if norm else {}
+    d, _ = kernels._gemv_desc(w, xd, out_f32=True, **kw)
+    plan = (C.c_int32 * 7)()
+    hip.call("mi_gemv_plan", C.byref(d), plan)
+    assert plan[0] == (3 if big else 1)
+    xin = rbf(x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + 1e-6) * nw) if norm else x
+    ref = ON.matmul_acc(xin, _dequant(block))
+    ref = np.tile(ref, (1, rep))[:, :n]
+    for ws in (None, torch.zeros(1024, dtype=torch.uint8, device="cuda")):
+        got = kernels.gemv(w, xd, out_f32=True, workspace=ws, **kw).cpu().numpy()
+        chk = check_against_oracle(got, ref)
+        assert (chk.ok_rounded() if norm else chk.ok()) and chk.within, (fmt, big, norm, chk)
+
+
 def test_fp8_dequant_every_code(torch_gpu):
     """Every finite E4M3 code (signed zero, subnormals, ±448) decodes bit-exactly; the tensor scale multiplies once."""
     from monolith_mi355 import kernels
