@@ -1043,15 +1043,18 @@ void gemv_rowp(Args a) {
   }
 }
 
-// ---- gemv_rowm: 3 <= M <= 16, NVFP4, FP8 and INT4 ---------------------------------------------------------------
+// ---- gemv_rowm: 2 <= M <= 16, every format ---------------------------------------------------------------------------
 // The gemv_row wave layout on the matrix cores, over several tiles per workgroup. Workgroup = S waves over tiles
 // blockIdx.x + j·G (j < ntl) and K split blockIdx.z; wave w owns a 512-column slice (4 NVFP4 / 8 FP8 chunks) of
 // every one of them. The
 // wave's activations for those chunks stay in VGPRs for the whole launch as the F16 A operands of
 // v_mfma_f32_16x16x32_f16 (token = A row; each token power-of-two scaled into F16 range over the wave's slice;
 // a fused input norm runs as its own launch before, see wants_prenorm); the weights are the B operand, decoded exactly to F16. Each wave
-// keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5) and issues the next as soon
-// as one is consumed. FP8 takes BF16 operands instead (its codes are exact BF16, the activations as they are). A
+// keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5;
+// BF16 one, its tile is 16 chunks) and issues the next as soon
+// as one is consumed. FP8 and BF16 take BF16 operands instead (their weights
+// are exact BF16, the activations as they are): BF16 8192 x 4096 at M = 3 / 8 / 16 22.3 / 22.5 / 23.2 us on gemv_tk, 13.5 /
+// 14.0 / 14.8 here. A
 // tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to exact F16
 // integers, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
 // scaled and offset by its (scale, bias) pair with the token's Σx over the group (held per lane for the launch).
@@ -1060,10 +1063,10 @@ constexpr int ROWM_SLD = 1024 + 16;             // bytes of a staged activation 
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 template <int FMT>
 __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
-  constexpr int KC = chunk_cols(FMT), KW = 512 / KC;   // a wave's slice is 512 columns: 4 NVFP4 / INT4, 8 FP8 chunks
+  constexpr int KC = chunk_cols(FMT), KW = 512 / KC;   // a wave's slice is 512 columns: 4 NVFP4 / INT4, 8 FP8, 16 BF16 chunks
   constexpr int SPC = KC / 32;                  // MFMA steps per chunk: the lane's KC/4 columns, 8 per step
-  static_assert(FMT == FMT_NVFP4 || FMT == FMT_FP8 || FMT == FMT_INT4, "gemv_rowm: NVFP4, FP8 or INT4");
-  constexpr bool I4 = FMT == FMT_INT4, F8 = FMT == FMT_FP8;
+  // BA: BF16 operands, the activations as they are (FP8 codes and BF16 weights are exact BF16)
+  constexpr bool I4 = FMT == FMT_INT4, BA = FMT == FMT_FP8 || FMT == FMT_BF16;
   constexpr int UB = I4 ? UNIT_Q : 1024;        // bytes from one chunk's codes to the next
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1102,7 +1105,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     for (int r = 0; r < 4; ++r) x[r] = *reinterpret_cast<const uint4*>(xbase + (long long)min(4 * grp + r, cnt - 1) * a.ldx);
   };
   uint4 xr[4], xn[4], xa[KW][SPC];
-  if constexpr (F8) {
+  if constexpr (BA) {
     const uint16_t* xrow = a.x + (long long)min(m_row, cnt - 1) * a.ldx + c0 * KC;
 #pragma unroll
     for (int cc = 0; cc < KW; ++cc)
@@ -1119,7 +1122,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   const long long c0_off = FMT == FMT_NVFP4 ? nv_code_off(c0) : (long long)c0 * unit_bytes(FMT);
   // NVFP4 / FP8 keep two tiles in flight per wave (the 12-wave workgroup leaves 168 VGPRs a lane); INT4's Σx
   // terms leave room for one
-  constexpr int DEPTH = I4 ? 1 : 2;
+  constexpr int DEPTH = I4 || FMT == FMT_BF16 ? 1 : 2;
   uint2 sb0[I4 ? KW : 1], sb1[I4 ? KW : 1];     // INT4: the (scale, bias) pairs of row m_row's two groups per chunk
   auto issue = [&](uint4 (&u)[KW], uint4& sv, uint2 (&sb)[I4 ? KW : 1], int j) {
     const uint8_t* tbase = wmat + (long long)tile_of(j) * a.tile_stride;
@@ -1152,10 +1155,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   for (int cc = 0; cc < KW; ++cc)               // padding tokens: zero operands
 #pragma unroll
     for (int s = 0; s < SPC; ++s)
-      if (!F8 || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
+      if (!BA || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
   float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};       // the lane's output tokens are 4g + i: their 2^p
 #pragma unroll 1
-  for (int grp = 0; !F8 && grp < ng; ++grp) {
+  for (int grp = 0; !BA && grp < ng; ++grp) {
     float psr[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1257,6 +1260,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
           acc[i] = fmaf(sca, da[i], fmaf(bia, sxa[i], acc[i]));
           acc[i] = fmaf(scb, db[i], fmaf(bib, sxb[i], acc[i]));
         }
+      } else if constexpr (FMT == FMT_BF16) {
+        const bf16x8 bv = __builtin_bit_cast(bf16x8, u[cc]);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[cc][0]), bv, acc, 0, 0, 0);
+        continue;                               // no decode: nothing to keep apart
       } else {                                  // FP8: the lane's 16 codes, 8 per step
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -1269,7 +1276,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     float* rp = red + wave * a.row_ld + jt * 256;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      rp[(4 * g + i) * 16 + m_row] = active ? (F8 ? acc[i] : acc[i] * (I4 ? ps[i] * 0x1p24f : ps[i])) : 0.0f;
+      rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : acc[i] * (I4 ? ps[i] * 0x1p24f : ps[i])) : 0.0f;
   };
   if constexpr (DEPTH == 1) {
     for (int j = 0; j < ntl; ++j) {
@@ -2175,6 +2182,7 @@ int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
   }
   int n = 0;
   const void* kern = fmt == FMT_FP8    ? reinterpret_cast<const void*>(gemv_rowm<FMT_FP8>)
+                     : fmt == FMT_BF16 ? reinterpret_cast<const void*>(gemv_rowm<FMT_BF16>)
                      : fmt == FMT_INT4 ? reinterpret_cast<const void*>(gemv_rowm<FMT_INT4>)
                                        : reinterpret_cast<const void*>(gemv_rowm<FMT_NVFP4>);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, threads, lds) !=
@@ -2189,7 +2197,7 @@ int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
 
 Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   Plan best{};
-  if ((d->format != FMT_NVFP4 && d->format != FMT_FP8 && d->format != FMT_INT4) || d->groups || d->gnorm_w || d->norm_w ||
+  if (d->groups || d->gnorm_w || d->norm_w ||
       d->m < 2 || d->m > 16 ||
       (d->format == FMT_NVFP4 && chunks % 4))     // NVFP4 slices start on half scale groups
     return best;
@@ -2252,11 +2260,11 @@ bool wants_prenorm(const mi_gemv_desc* d) {
 // stream, the matrix cores take any M at the price of one, and the norm's launch costs less than normalizing two rows
 // in every workgroup. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 42.9 → 23.3 us, without 29.0 →
 // 20.7, in_proj with the norm 23.4 → 15.5, down 17.0 → 15.0, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
-// MB, norm) 11.5 → 10.8; below that gemv_row wins: N = 12288, K = 2048 (14.2 MB, norm) 7.9 against 8.1, FP8 4096 x 4096
+// MB, norm) 11.5 → 10.8, BF16 8192 x 4096 17.5 → 13.5; below that gemv_row wins: N = 12288, K = 2048 (14.2 MB, norm) 7.9 against 8.1, FP8 4096 x 4096
 // (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4.
 constexpr size_t kRowmTwoBytes = 20u << 20;
 bool rowm_at_two(const mi_gemv_desc* d) {
-  return d->m == 2 && !d->groups && !d->gnorm_w && !d->conv_w && d->format != FMT_BF16 &&
+  return d->m == 2 && !d->groups && !d->gnorm_w && !d->conv_w &&
          (size_t)((d->n + 15) / 16) * (size_t)tile_bytes(d->format, d->k / chunk_cols(d->format)) >= kRowmTwoBytes &&
          !getenv("MI_GEMV_KERNEL") && !getenv("MI_GEMV_ROW");
 }
@@ -2332,11 +2340,10 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
   }
   // Grouped (MoE) NVFP4 launches at M >= 3: routing spreads the tokens over the experts, so a group holds one or
   // two pairs (the shared expert's group all of them): gemv_row takes them two per workgroup (grid z: the passes)
-  // instead of gemv_tk padding every group to 16 MFMA rows. A small BF16 matrix (the MoE router, 1 MB) the same
-  // way, two tokens per workgroup: its passes re-read it from the caches, and no split-K reduction launch follows.
-  // (NVFP4 stays on gemv_rowm: the attention o_proj, 8.8 MB, measured 11.8 → 10.5–10.8 µs alone but no faster in
-  // the layer; out_proj, 17.7 MB, and q|k|v, 20 MB, are slower with passes)
-  const bool small = !d->groups && !d->gnorm_w && fmt == FMT_BF16 && (size_t)d->n * d->k * 2 <= (8u << 20);
+  // instead of gemv_tk padding every group to 16 MFMA rows. A BF16 matrix of at most 256 KB the same way, two
+  // tokens per workgroup (64 x 2048 at M = 8 / 16 4.3 / 4.3 us against gemv_rowm's 4.4 / 4.9; the MoE router, 257 x 2048,
+  // 5.0 / 6.0 against 4.4 / 5.1)
+  const bool small = !d->groups && !d->gnorm_w && fmt == FMT_BF16 && (size_t)d->n * d->k * 2 <= (256u << 10);
   if (rows > 2 && ((d->groups && fmt == FMT_NVFP4) || small) && !pin_tk && !pin_rowm &&
       !(getenv("MI_GEMV_PASSES") && getenv("MI_GEMV_PASSES")[0] == '0')) {       // =0: the earlier plans (A/B)
     Plan p = plan_row(d, fmt, chunks, 2, n_tiles, groups);
@@ -2401,13 +2408,11 @@ void launch_reduce(const Args& a, hipStream_t s) {
 
 template <int FMT>
 void launch(const Args& a, const Plan& p, int groups, hipStream_t s) {
-  if constexpr (FMT == FMT_NVFP4 || FMT == FMT_FP8 || FMT == FMT_INT4) {
-    if (p.kernel == 3) {
-      allow_lds(gemv_rowm<FMT>);
-      hipLaunchKernelGGL(gemv_rowm<FMT>, dim3(p.G, 1, p.ks), dim3(64 * p.S), p.lds_bytes, s, a);
-      if (p.ks > 1) launch_reduce(a, s);
-      return;
-    }
+  if (p.kernel == 3) {
+    allow_lds(gemv_rowm<FMT>);
+    hipLaunchKernelGGL(gemv_rowm<FMT>, dim3(p.G, 1, p.ks), dim3(64 * p.S), p.lds_bytes, s, a);
+    if (p.ks > 1) launch_reduce(a, s);
+    return;
   }
   if (p.kernel == 1) {
     const dim3 g(p.G, groups, p.passes > 1 ? p.passes : p.ks);

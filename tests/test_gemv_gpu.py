@@ -272,7 +272,7 @@ def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch
     assert chk.ok_rounded() and chk.within, (mtok, n, k, plan, epi, chk)
 
 
-@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3"])
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("mtok", [3, 4, 5, 8, 9, 13, 16])
 @pytest.mark.parametrize("n,k", [(24, 128), (4117, 640), (40, 6656)])
 def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
@@ -293,7 +293,7 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
         assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
 
 
-@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3"])
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("big", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
 def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
@@ -304,7 +304,7 @@ def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
     from monolith_mi355.runtime import hip
     torch = torch_gpu
     k = 1024
-    per_row = {"nvfp4": 576, "int4_affine": 576, "fp8_e4m3": 1024}[fmt]
+    per_row = {"nvfp4": 576, "int4_affine": 576, "fp8_e4m3": 1024, "bf16": 2048}[fmt]
     n = ((20 << 20) // (per_row * 16) + (1 if big else -1)) * 16
     block = _matrix(fmt, 512, k, rng)                       # 512 random rows down the matrix
     rep = -(-n // 512)
