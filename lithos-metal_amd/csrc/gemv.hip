@@ -521,12 +521,13 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
   float acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
-  auto slice_chunk = [&](int cc) {
+  auto slice_chunk = [&](int cc, auto tokens) {
+    constexpr int TT = decltype(tokens)::value;   // tokens of this workgroup: MT, or one of two
     const uint32_t dw[4] = {u[cc].q.x, u[cc].q.y, u[cc].q.z, u[cc].q.w};
     if constexpr (FMT == FMT_NVFP4) {
-      uint4 xq[MT][4];
+      uint4 xq[TT][4];
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
+      for (int t = 0; t < TT; ++t)
 #pragma unroll
         for (int s = 0; s < 4; ++s) xq[t][s] = *reinterpret_cast<const uint4*>(xs + (size_t)t * ld + cc * 128 + 32 * g + 8 * s);
       // chunk in its group: KW >= 8 slices start on a group, KW = 4 slices on one of its halves (c0 % 4 == 0)
@@ -541,43 +542,43 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
                              nv_mant(u1)};
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        float part[MT];
+        float part[TT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) part[t] = 0.0f;
+        for (int t = 0; t < TT; ++t) part[t] = 0.0f;
 #pragma unroll
         for (int s = 2 * b; s < 2 * b + 2; ++s)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const bf16x2 w2 = cvt_fp4x2_bf16(dw[s], e[b], j);
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
+            for (int t = 0; t < TT; ++t) {
               const uint32_t xw = j == 0 ? xq[t][s].x : j == 1 ? xq[t][s].y : j == 2 ? xq[t][s].z : xq[t][s].w;
               part[t] = __builtin_amdgcn_fdot2_f32_bf16(w2, __builtin_bit_cast(bf16x2, xw), part[t], false);
             }
           }
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = fmaf(part[t], mant[b], acc[t]);
+        for (int t = 0; t < TT; ++t) acc[t] = fmaf(part[t], mant[b], acc[t]);
       }
     } else if constexpr (FMT == FMT_INT4) {
-      uint4 xq[MT][4];
-      float sa[MT], sb[MT];
+      uint4 xq[TT][4];
+      float sa[TT], sb[TT];
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
+      for (int t = 0; t < TT; ++t) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) xq[t][s] = *reinterpret_cast<const uint4*>(xs + (size_t)t * ld + cc * 128 + 32 * s + 8 * g);
         sa[t] = seg[(t * KW + cc) * 8 + g * 2];
         sb[t] = seg[(t * KW + cc) * 8 + g * 2 + 1];
       }
-      float d[2][MT];
+      float d[2][TT];
 #pragma unroll
-      for (int t = 0; t < MT; ++t) d[0][t] = d[1][t] = 0.0f;
+      for (int t = 0; t < TT; ++t) d[0][t] = d[1][t] = 0.0f;
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t w2 = ((dw[s] >> (4 * j)) & 0x000F000Fu) | 0x43004300u;   // BF16 (128 + n_j, 128 + n_j+4)
 #pragma unroll
-          for (int t = 0; t < MT; ++t) {
+          for (int t = 0; t < TT; ++t) {
             const uint32_t xw = j == 0 ? xq[t][s].x : j == 1 ? xq[t][s].y : j == 2 ? xq[t][s].z : xq[t][s].w;
             d[s >> 1][t] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w2), __builtin_bit_cast(bf16x2, xw),
                                                            d[s >> 1][t], false);
@@ -586,14 +587,14 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
       const float sca = bf16_bits_to_f32(u[cc].sb.x & 0xFFFFu), bia = bf16_bits_to_f32(u[cc].sb.x >> 16);
       const float scb = bf16_bits_to_f32(u[cc].sb.y & 0xFFFFu), bib = bf16_bits_to_f32(u[cc].sb.y >> 16);
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
+      for (int t = 0; t < TT; ++t) {
         acc[t] = fmaf(sca, fmaf(-128.0f, sa[t], d[0][t]), fmaf(bia, sa[t], acc[t]));
         acc[t] = fmaf(scb, fmaf(-128.0f, sb[t], d[1][t]), fmaf(bib, sb[t], acc[t]));
       }
     } else if constexpr (FMT == FMT_FP8) {
-      uint4 xq[MT][2];                      // the lane's 16 columns 64·cc + 16·g + [0, 16)
+      uint4 xq[TT][2];                      // the lane's 16 columns 64·cc + 16·g + [0, 16)
     #pragma unroll
-      for (int t = 0; t < MT; ++t)
+      for (int t = 0; t < TT; ++t)
     #pragma unroll
         for (int h = 0; h < 2; ++h) xq[t][h] = *reinterpret_cast<const uint4*>(xs + (size_t)t * ld + cc * 64 + 16 * g + 8 * h);
     #pragma unroll
@@ -602,7 +603,7 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
         for (int hi = 0; hi < 2; ++hi) {
           const bf16x2 w2 = cvt_fp8x2_bf16(dw[q], hi);   // columns 4q + 2hi, +1 of the lane's 16
     #pragma unroll
-          for (int t = 0; t < MT; ++t) {
+          for (int t = 0; t < TT; ++t) {
             const uint4 xv4 = xq[t][q >> 1];
             const int e = 2 * (q & 1) + hi;
             const uint32_t xw = e == 0 ? xv4.x : e == 1 ? xv4.y : e == 2 ? xv4.z : xv4.w;
@@ -610,22 +611,29 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
           }
         }
     } else {
-      uint4 xq[MT];
+      uint4 xq[TT];
 #pragma unroll
-      for (int t = 0; t < MT; ++t) xq[t] = *reinterpret_cast<const uint4*>(xs + (size_t)t * ld + cc * 32 + 8 * g);
+      for (int t = 0; t < TT; ++t) xq[t] = *reinterpret_cast<const uint4*>(xs + (size_t)t * ld + cc * 32 + 8 * g);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
+        for (int t = 0; t < TT; ++t) {
           const uint32_t xw = j == 0 ? xq[t].x : j == 1 ? xq[t].y : j == 2 ? xq[t].z : xq[t].w;
           acc[t] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, dw[j]), __builtin_bit_cast(bf16x2, xw),
                                                    acc[t], false);
         }
     }
   };
+  // a grouped launch's records of two pairs mostly hold one (64 picks over 256 experts): half the dot products then
+  if (MT > 1 && cnt == 1) {
 #pragma unroll
-  for (int cc = 0; cc < KW; ++cc)
-    if (cc < kw) slice_chunk(cc);
+    for (int cc = 0; cc < KW; ++cc)
+      if (cc < kw) slice_chunk(cc, std::integral_constant<int, 1>{});
+  } else {
+#pragma unroll
+    for (int cc = 0; cc < KW; ++cc)
+      if (cc < kw) slice_chunk(cc, std::integral_constant<int, MT>{});
+  }
 
   // ---- the four k-groups of each row, then the K slices in wave order, then the epilogue ------------------------
 #pragma unroll
