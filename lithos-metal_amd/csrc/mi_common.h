@@ -81,16 +81,27 @@ __device__ __forceinline__ float max16(float v) {
   return v;
 }
 
-// the largest of the wave's integers, in every lane
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xF, 0xF, true));
-  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppXor2, 0xF, 0xF, true));
-  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppHalfMirror, 0xF, 0xF, true));
-  v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppMirror, 0xF, 0xF, true));
+// the largest / smallest of the wave's integers, in every lane (the exchange folds into the instruction, where a float
+// maximum takes three: half the chain of wave_max)
+template <typename T, typename F>
+__device__ __forceinline__ T wave_fold(T v, F f) {
+  v = f(v, (T)__builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xF, 0xF, true));
+  v = f(v, (T)__builtin_amdgcn_mov_dpp((int)v, kDppXor2, 0xF, 0xF, true));
+  v = f(v, (T)__builtin_amdgcn_mov_dpp((int)v, kDppHalfMirror, 0xF, 0xF, true));
+  v = f(v, (T)__builtin_amdgcn_mov_dpp((int)v, kDppMirror, 0xF, 0xF, true));
   const auto r = __builtin_amdgcn_permlane16_swap((int)v, (int)v, false, false);
-  v = max((uint32_t)r[0], (uint32_t)r[1]);
+  v = f((T)r[0], (T)r[1]);
   const auto q = __builtin_amdgcn_permlane32_swap((int)v, (int)v, false, false);
-  return max((uint32_t)q[0], (uint32_t)q[1]);
+  return f((T)q[0], (T)q[1]);
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  return wave_fold(v, [](uint32_t a, uint32_t b) { return max(a, b); });
+}
+__device__ __forceinline__ int wave_max_i32(int v) {
+  return wave_fold(v, [](int a, int b) { return max(a, b); });
+}
+__device__ __forceinline__ int wave_min_i32(int v) {
+  return wave_fold(v, [](int a, int b) { return min(a, b); });
 }
 
 // v(l) + v(l ^ 16) and v(l) + v(l ^ 32): a swap leaves each lane holding its own value in one half of the pair and

@@ -37,25 +37,31 @@ __device__ __forceinline__ void route_topk_n(const uint16_t* logits, int E, int 
     s += v[i];
   }
   s = wave_sum(s);
+  // the probabilities as integers: not negative, so their bits order as they do, and -1 marks an absent or taken expert
+  // (a NaN is absent too). A pick is two integer folds over the wave; as float maxima the k picks were most of the launch
+  int b[NPL];
 #pragma unroll
-  for (int i = 0; i < NPL; ++i) v[i] = lane + 64 * i < E ? v[i] / s : -1.0f;   // -1: absent or taken
+  for (int i = 0; i < NPL; ++i) {
+    const float p = v[i] / s;
+    b[i] = lane + 64 * i < E && p >= 0.0f ? __float_as_int(p) : -1;
+  }
   float wsum = 0.0f;
   for (int r = 0; r < k; ++r) {
-    float best = -1.0f;
-    int bi = 1 << 20;
+    int best = -1, bi = 1 << 20;
 #pragma unroll
     for (int i = 0; i < NPL; ++i)
-      if (v[i] > best) { best = v[i]; bi = lane + 64 * i; }        // strictly greater: the lane's lowest index
-    const float gmax = wave_max(best);
-    const int e = (int)-wave_max(-(best == gmax ? (float)bi : (float)(1 << 20)));
-    if (e >= E) {                     // no finite probability left (NaN logits): no expert, weight 0
+      if (b[i] > best) { best = b[i]; bi = lane + 64 * i; }        // strictly greater: the lane's lowest index
+    const int top = wave_max_i32(best);
+    const int e = wave_min_i32(best == top ? bi : 1 << 20);
+    if (top < 0 || e >= E) {          // no finite probability left (NaN logits): no expert, weight 0
       ce[r] = -1;
       cw[r] = 0.0f;
       continue;
     }
 #pragma unroll
     for (int i = 0; i < NPL; ++i)
-      if (lane + 64 * i == e) v[i] = -1.0f;
+      if (lane + 64 * i == e) b[i] = -1;
+    const float gmax = __int_as_float(top);
     ce[r] = e;
     cw[r] = gmax;
     wsum += gmax;
