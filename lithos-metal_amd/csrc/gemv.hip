@@ -2267,9 +2267,10 @@ bool wants_prenorm(const mi_gemv_desc* d) {
 // Two tokens over a large weight stream run on gemv_rowm: gemv_row's dot products for two tokens (VALU) fall behind the
 // stream, the matrix cores take any M at the price of one, and the norm's launch costs less than normalizing two rows
 // in every workgroup. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 42.9 → 23.3 us, without 29.0 →
-// 20.7, in_proj with the norm 23.4 → 15.5, down 17.0 → 15.0, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
+// 20.7, in_proj with the norm 23.4 → 15.5, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
 // MB, norm) 11.5 → 10.8, BF16 8192 x 4096 17.5 → 13.5; below that gemv_row wins: N = 12288, K = 2048 (14.2 MB, norm) 7.9 against 8.1, FP8 4096 x 4096
-// (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4.
+// (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4. A K that gemv_rowm would split (over 6144) stays on
+// gemv_row, which folds its splits in the kernel and needs no partials for them.
 constexpr size_t kRowmTwoBytes = 20u << 20;
 bool rowm_at_two(const mi_gemv_desc* d) {
   return d->m == 2 && !d->groups && !d->gnorm_w && !d->conv_w &&
@@ -2284,7 +2285,7 @@ Plan make_plan(const mi_gemv_desc* d, bool two = true) {
     plain.norm_w = nullptr;
     Plan p = plan_rowm(&plain, d->k / chunk_cols(d->format), (d->n + 15) / 16);
     p.prenorm = p.kernel != 0 && d->norm_w;
-    if (p.kernel) return p;
+    if (p.kernel && p.ks == 1) return p;
   }
   if (d->conv_w) {                              // the conv epilogue lives in gemv_row: one tile per workgroup
     Plan p = make_plan_fused(d);
