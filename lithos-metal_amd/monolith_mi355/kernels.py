@@ -18,9 +18,15 @@ from .formats import pack as _pack
 from .runtime import hip
 
 
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
 def _check_flag(flag, name, what="done"):
@@ -69,10 +75,10 @@ def upload(specs, device="cuda", row_scales=None) -> PackedWeight:
 
 
 def _bf16_2d(t, name, aligned=True):
-    torch = _torch()
-    if t.dtype != torch.bfloat16 or t.dim() != 2 or t.stride(1) != 1:
+    s = t.stride()
+    if t.dtype != _torch().bfloat16 or len(s) != 2 or s[1] != 1:
         raise ValueError(f"{name}: expected a row-major 2-D bfloat16 tensor, got {t.dtype} {tuple(t.shape)}")
-    if aligned and (t.data_ptr() % 16 or t.stride(0) % 8):
+    if aligned and (t.data_ptr() % 16 or s[0] % 8):
         raise ValueError(f"{name}: needs 16-byte alignment and a row stride multiple of 8")
 
 
@@ -164,15 +170,25 @@ def _gemv_desc(w: PackedWeight, x, *, epilogue=None, residual=None, norm_w=None,
         _bf16_2d(gz, "gemv gated_norm z")
         if gz.shape[0] < m or gz.shape[1] < k:
             raise ValueError("gemv: gated_norm z too small")
-    d = hip.MiGemvDesc(format=hip.MI_FMT[w.format], n=w.n, k=w.k, m=m, w=hip.ptr(w.data),
-                       row_scale=hip.ptr(w.row_scale), x=hip.ptr(x), ldx=x.stride(0), y=hip.ptr(out),
-                       ldy=out.stride(0), epilogue=hip.MI_EPI[epilogue],
-                       residual=hip.ptr(residual) if epilogue == "residual" else 0,
-                       ldr=residual.stride(0) if epilogue == "residual" else 0, norm_w=hip.ptr(norm_w), eps=eps,
-                       groups=0, max_groups=0, top_k=0, x_per_slot=0,
-                       workspace=hip.ptr(workspace), workspace_bytes=0 if workspace is None else workspace.numel(),
-                       out_f32=int(out_f32), gnorm_w=hip.ptr(gw), gnorm_z=hip.ptr(gz),
-                       ld_gnorm_z=gz.stride(0) if gz is not None else 0, gnorm_eps=geps)
+    d = hip.MiGemvDesc()                    # zeros: only what this call uses is set (a third of the wrapper's time)
+    d.format, d.n, d.k, d.m = hip.MI_FMT[w.format], w.n, k, m
+    d.w, d.x, d.y = hip.ptr(w.data), x.data_ptr(), out.data_ptr()
+    d.ldx, d.ldy, d.eps = x.stride(0), out.stride(0), eps
+    if w.row_scale is not None:
+        d.row_scale = hip.ptr(w.row_scale)
+    if epilogue is not None:
+        d.epilogue = hip.MI_EPI[epilogue]
+        if epilogue == "residual":
+            d.residual, d.ldr = residual.data_ptr(), residual.stride(0)
+    if norm_w is not None:
+        d.norm_w = norm_w.data_ptr()
+    if workspace is not None:
+        d.workspace, d.workspace_bytes = workspace.data_ptr(), workspace.numel()
+    if out_f32:
+        d.out_f32 = 1
+    if gated_norm is not None:
+        d.gnorm_w, d.gnorm_z = gw.data_ptr(), gz.data_ptr()
+        d.ld_gnorm_z, d.gnorm_eps = gz.stride(0), geps
     return d, out
 
 

@@ -260,7 +260,7 @@ def last_error() -> str:
 
 
 def call(name: str, *args) -> int:
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
         raise MiError(f"{name} failed ({rc}): {last_error()}")
     return rc
@@ -286,10 +286,12 @@ def stream_handle(stream=None) -> Optional[int]:
     if stream is None:
         try:
             import torch
-            if torch.cuda.is_available():
-                return int(torch.cuda.current_stream().cuda_stream)
         except ImportError:
-            pass
+            return None
+        if torch.cuda.is_initialized():     # the handle itself: making a Stream object of it takes longer than a launch's checks
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        if torch.cuda.is_available():
+            return int(torch.cuda.current_stream().cuda_stream)
         return None
     if isinstance(stream, int):
         return stream
