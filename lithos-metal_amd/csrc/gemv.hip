@@ -308,10 +308,12 @@ __device__ __forceinline__ void load_chunk(Units<FMT>& u, const uint8_t* tb, int
 // ---- gemv_row: M <= 2 ------------------------------------------------------------------------------------------
 // Workgroup = one 16-row tile (blockIdx.x) of one group (blockIdx.y, MoE); wave w = K slice [w·KW, w·KW + KW).
 // LDS: per wave xs[MT][row_ld] (INT4: then seg[MT][KW][8]) | stat[S][2] | red[S][MT][16].
-// CONV: the launch carries the GDN conv epilogue (a separate instantiation: its registers and code stay out of the
-// plain GEMV, whose occupancy they would otherwise cut).
-template <int FMT, int MT, int KW, bool CONV>
+// ROW_CONV: the launch carries the GDN conv epilogue; ROW_PAIRS: a grouped launch of two pairs a record (separate
+// instantiations: their registers and code stay out of the plain GEMV).
+enum { ROW_PLAIN, ROW_CONV, ROW_PAIRS };
+template <int FMT, int MT, int KW, int MODE>
 __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
+  constexpr bool CONV = MODE == ROW_CONV;
   constexpr int KC = chunk_cols(FMT);
   constexpr int NPL = MT * KW * KC / 8 / 64 > 0 ? MT * KW * KC / 8 / 64 : 1;   // activation vectors per lane
   constexpr int NG = FMT == FMT_NVFP4 ? (KW + 7) / 8 : 0;                         // scale pieces per wave
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(KW == 16 ? 640 : 1024) void gemv_row(Args a) {
     }
   };
   // a grouped launch's records of two pairs mostly hold one (64 picks over 256 experts): half the dot products then
-  if (MT > 1 && cnt == 1) {
+  if (MODE == ROW_PAIRS && cnt == 1) {
 #pragma unroll
     for (int cc = 0; cc < KW; ++cc)
       if (cc < kw) slice_chunk(cc, std::integral_constant<int, 1>{});
@@ -2207,7 +2209,7 @@ Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   Plan best{};
   if (d->groups || d->gnorm_w || d->norm_w ||
       d->m < 2 || d->m > 16 ||
-      (d->format == FMT_NVFP4 && chunks % 4))     // NVFP4 slices start on half scale groups
+      (d->format == FMT_NVFP4 && chunks < 4))     // less than a slice of K: one short stream a tile, gemv_tk's
     return best;
   const int kw = 512 / chunk_cols(d->format);    // chunks per wave (512 columns)
   int ks = (chunks + 12 * kw - 1) / (12 * kw);   // at most 12 waves: the kernel's VGPR budget is 3 waves per SIMD
@@ -2392,9 +2394,9 @@ void launch_tk_d(const Args& a, const Plan& p, dim3 g, hipStream_t s) {
 template <int FMT, int MT, int KW>
 void launch_row_kw(const Args& a, const Plan& p, dim3 g, hipStream_t s) {
   if (MT == 1 && p.rt > 1) { allow_lds(gemv_rowp<FMT, 1, KW>); hipLaunchKernelGGL((gemv_rowp<FMT, 1, KW>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
-  else if (a.conv_w) {
-    if constexpr (MT <= 2) { allow_lds(gemv_row<FMT, MT, KW, true>); hipLaunchKernelGGL((gemv_row<FMT, MT, KW, true>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
-  } else { allow_lds(gemv_row<FMT, MT, KW, false>); hipLaunchKernelGGL((gemv_row<FMT, MT, KW, false>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
+  else if (a.conv_w) { allow_lds(gemv_row<FMT, MT, KW, ROW_CONV>); hipLaunchKernelGGL((gemv_row<FMT, MT, KW, ROW_CONV>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
+  else if (MT == 2 && a.groups) { allow_lds(gemv_row<FMT, 2, KW, ROW_PAIRS>); hipLaunchKernelGGL((gemv_row<FMT, 2, KW, ROW_PAIRS>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
+  else { allow_lds(gemv_row<FMT, MT, KW, ROW_PLAIN>); hipLaunchKernelGGL((gemv_row<FMT, MT, KW, ROW_PLAIN>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
 }
 
 template <int FMT, int MT>

@@ -274,7 +274,7 @@ def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("mtok", [3, 4, 5, 8, 9, 13, 16])
-@pytest.mark.parametrize("n,k", [(24, 128), (4117, 640), (40, 6656)])
+@pytest.mark.parametrize("n,k", [(24, 128), (4117, 640), (56, 896), (33, 1792), (40, 6656)])
 def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
     """Every remainder of the four rows staged at a time, a slice of one chunk, one more tile than workgroups, two K
     splits; a row of zeros, one scaled by 2^60 and one by 2^-60 (each row's own power-of-two prescale): every row
