@@ -2270,13 +2270,17 @@ bool wants_prenorm(const mi_gemv_desc* d) {
 // stream, the matrix cores take any M at the price of one, and the norm's launch costs less than normalizing two rows
 // in every workgroup. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 42.9 → 23.3 us, without 29.0 →
 // 20.7, in_proj with the norm 23.4 → 15.5, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
-// MB, norm) 11.5 → 10.8, BF16 8192 x 4096 17.5 → 13.5; below that gemv_row wins: N = 12288, K = 2048 (14.2 MB, norm) 7.9 against 8.1, FP8 4096 x 4096
+// MB, norm) 11.5 → 10.8, BF16 8192 x 4096 17.5 → 13.5. Below, and for a short K (few waves share a workgroup's
+// activations), gemv_row wins or ties: N = 34816 with the norm K = 1024 / 1536 / 2048 / 3072 9.8 / 12.7 / 14.3 / 24.4 against
+// 10.6 / 12.5 / 13.3 / 16.8 us, without it 7.9 / 9.3 / 10.7 / 16.6 against 8.3 / 9.9 / 10.9 / 14.1, INT4 K = 2048 16.0
+// against 18.2, FP8 8192 x 4096 (33.6 MB, norm) 10.7 against 10.9, BF16 12288 x 2048 13.4 against 13.1, FP8 4096 x 4096
 // (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4. A K that gemv_rowm would split (over 6144) stays on
 // gemv_row, which folds its splits in the kernel and needs no partials for them.
 constexpr size_t kRowmTwoBytes = 20u << 20;
 bool rowm_at_two(const mi_gemv_desc* d) {
-  return d->m == 2 && !d->groups && !d->gnorm_w && !d->conv_w &&
-         (size_t)((d->n + 15) / 16) * (size_t)tile_bytes(d->format, d->k / chunk_cols(d->format)) >= kRowmTwoBytes &&
+  const size_t least = d->format == FMT_FP8 ? 2 * kRowmTwoBytes : kRowmTwoBytes;
+  return d->m == 2 && d->k >= (d->format == FMT_BF16 ? 2048 : 3072) && !d->groups && !d->gnorm_w && !d->conv_w &&
+         (size_t)((d->n + 15) / 16) * (size_t)tile_bytes(d->format, d->k / chunk_cols(d->format)) >= least &&
          !getenv("MI_GEMV_KERNEL") && !getenv("MI_GEMV_ROW");
 }
 

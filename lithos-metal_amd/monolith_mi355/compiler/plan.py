@@ -18,7 +18,7 @@ terms, each pass checking the pattern it folds and leaving anything else as it i
 * ``fold_norm_apply`` — a ``norm_apply`` whose output feeds only GEMVs becomes their fused input norm;
 * ``fuse_gdn`` — ``gdn_mixer`` + its ``gdn_norm`` become one ``mi_gdn_step``; at T ≤ 2 the norm moves onto the
   output projection's load (``defer``), as the hand-built layer does;
-* ``fold_gdn_conv`` — at T = 1 the GDN short conv runs in the input projection's epilogue, and the step reads the
+* ``fold_gdn_conv`` — at T ≤ 2 the GDN short conv runs in the input projection's epilogue, and the step reads the
   convolved values;
 * ``fuse_gqa`` — ``gqa_decode`` + ``gqa_merge`` become one ``mi_gqa_decode`` (the merge and the gate inside);
 * ``fuse_shared_expert`` — a MoE block whose shared expert has the routed experts' shape and sits right after them
@@ -33,6 +33,7 @@ from dataclasses import dataclass, field
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
 from ..core.shapes import bind, step_bindings
+from ..formats.pack import two_tokens_on_matrix_cores
 
 
 @dataclass(eq=False)
@@ -303,12 +304,12 @@ def fuse_gdn(p: Plan, defer_max_t: int = 2) -> None:
 
 
 def fold_gdn_conv(p: Plan) -> None:
-    """At T = 1 the GDN short conv moves into the input projection's epilogue (``mi_gemv_desc.conv_*``): the GEMV
+    """At T <= 2 the GDN short conv moves into the input projection's epilogue (``mi_gemv_desc.conv_*``): the GEMV
     that produces the step's q|k|v rows convolves each of them where it is computed and writes the convolved values
     to a buffer the step reads (``mi_gdn_desc.pre``); the step then skips its conv section (≈ 4 µs of dependent
-    loads at one token). The commit pass of a speculative program keeps its own conv. At T = 2 the projection runs on the
-    matrix cores without it, as in the hand-built layer."""
-    if p.t > 1:
+    loads at one token). The commit pass of a speculative program keeps its own conv. At T = 2 a large
+    projection runs on the matrix cores without it, as in the hand-built layer."""
+    if p.t > 2:
         return
     for op in p.ops:
         if op.kind != "gdn_mixer":
@@ -319,6 +320,8 @@ def fold_gdn_conv(p: Plan) -> None:
         root, col = p.root(qkv_val)
         prod = next((o for o in p.ops if o.kind == "gemv" and o.outputs[0].name == root), None)
         if prod is None or prod.attrs.get("epilogue") is not None or prod.attrs.get("row_range") is not None:
+            continue
+        if p.t == 2 and two_tokens_on_matrix_cores(prod.inputs[1].format or "nvfp4", *p.shape(prod.inputs[1])[:2]):
             continue
         n_main = 1 + max(idx for idx, _, _ in ps.values())
         cs = op.inputs[n_main]

@@ -62,6 +62,13 @@ def pack_bytes(fmt: str, n: int, k: int) -> int:
     return -(-n // 16) * (k // chunk_cols(fmt)) * unit_bytes(fmt)
 
 
+def two_tokens_on_matrix_cores(fmt: str, n: int, k: int) -> bool:
+    """Whether a dense GEMV of two tokens runs on the matrix-core kernel (many weights, a long K in one split; the same
+    rule and its figures: ``csrc/gemv.hip`` ``rowm_at_two``); the Gated DeltaNet conv then stays out of its epilogue."""
+    least = (40 if fmt == "fp8_e4m3" else 20) << 20
+    return pack_bytes(fmt, n, k) >= least and (2048 if fmt == "bf16" else 3072) <= k <= 6144
+
+
 @dataclass
 class PackInfo:
     format: str

@@ -20,6 +20,7 @@ import numpy as np
 
 from . import kernels
 from .formats import device as DV
+from .formats.pack import two_tokens_on_matrix_cores
 
 
 def _torch():
@@ -31,10 +32,11 @@ def _torch():
 # persistent GEMV chain launch (kernels.gemv_chain) instead of one launch per GEMV. Off by default: at the 27B shapes
 # the chain measured slower (MLP 46–48 µs against 38–41 µs for the two launches)
 CHAIN_TAIL = os.environ.get("MI_LAYER_CHAIN", "0") == "1"
-# At one token the Gated DeltaNet short conv runs in the input projection's epilogue (each projection row of
+# At one or two tokens the Gated DeltaNet short conv runs in the input projection's epilogue (each projection row of
 # the q|k|v channels is convolved where it is produced) and the step reads the convolved values; MI_GDN_FOLD=0 keeps
-# the conv inside gdn_step (A/B comparisons). At two tokens the projection without the conv runs on the matrix cores and
-# the conv stays in the step: 27B layer 84.4 → 78.3 µs
+# the conv inside gdn_step (A/B comparisons). Two tokens over a large projection run on the matrix cores without the
+# conv, which stays in the step: 27B layer 84.4 → 78.3 µs; a small one keeps it (hidden 1408, 24 value heads 43.2 against
+# 44.5 µs)
 FOLD_CONV = os.environ.get("MI_GDN_FOLD", "1") != "0"
 
 
@@ -142,14 +144,15 @@ class GdnDecoderLayer:
         self._bufs: Dict[int, tuple] = {}
 
     def pre(self, m: int):
-        """The convolved q|k|v [m, conv_dim] the input projection writes when it runs the conv (m = 1)."""
+        """The convolved q|k|v [m, conv_dim] the input projection writes when it runs the conv (m <= 2)."""
         key = ("pre", m)
         if key not in self._bufs:
             self._bufs[key] = _torch().empty(m, self.conv_dim, dtype=_torch().bfloat16, device=self.rec_state.device)
         return self._bufs[key]
 
     def folds_conv(self, m: int, verify: bool = False) -> bool:
-        return FOLD_CONV and m == 1 and not verify
+        return FOLD_CONV and not verify and (m == 1 or (m == 2 and not two_tokens_on_matrix_cores(
+            self.w_in.packed.format, self.n_proj, self.hidden)))
 
     def buffers(self, m: int):
         torch = _torch()

@@ -297,15 +297,17 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
 @pytest.mark.parametrize("big", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
 def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
-    """Two tokens on either side of the weight bytes where gemv_rowm takes over (20 MiB): the plan, the rows against the
+    """Two tokens on either side of the weight bytes where gemv_rowm takes over (20 MiB, FP8 40): the plan, the rows against the
     oracle's float64 product, and a workspace too small for gemv_rowm's scratch (then gemv_row, the same gate)."""
     import ctypes as C
     from monolith_mi355 import kernels
     from monolith_mi355.runtime import hip
     torch = torch_gpu
-    k = 1024
-    per_row = {"nvfp4": 576, "int4_affine": 576, "fp8_e4m3": 1024, "bf16": 2048}[fmt]
-    n = ((20 << 20) // (per_row * 16) + (1 if big else -1)) * 16
+    from monolith_mi355.formats.pack import two_tokens_on_matrix_cores
+    k = 3072
+    per_row = {"nvfp4": 1728, "int4_affine": 1728, "fp8_e4m3": 3072, "bf16": 6144}[fmt]
+    n = (((40 if fmt == "fp8_e4m3" else 20) << 20) // (per_row * 16) + (1 if big else -1)) * 16
+    assert two_tokens_on_matrix_cores(fmt, n, k) == big
     block = _matrix(fmt, 512, k, rng)                       # 512 random rows down the matrix
     rep = -(-n // 512)
     m = {kk: (np.tile(v, (rep, 1))[:n].copy() if isinstance(v, np.ndarray) and v.ndim == 2 else v) for kk, v in block.items()}
@@ -320,7 +322,8 @@ def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
     xin = rbf(x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + 1e-6) * nw) if norm else x
     ref = ON.matmul_acc(xin, _dequant(block))
     ref = np.tile(ref, (1, rep))[:, :n]
-    for ws in (None, torch.zeros(1024, dtype=torch.uint8, device="cuda")):
+    small = torch.zeros(1024, dtype=torch.uint8, device="cuda")
+    for ws in (None,) if fmt == "bf16" else (None, small):   # BF16 at this K splits on gemv_row too: it needs partials
         got = kernels.gemv(w, xd, out_f32=True, workspace=ws, **kw).cpu().numpy()
         chk = check_against_oracle(got, ref)
         assert (chk.ok_rounded() if norm else chk.ok()) and chk.within, (fmt, big, norm, chk)
