@@ -8,7 +8,7 @@
 // MI355X design. The pack streams 16-row tiles in 128-column chunks; lane l of a wave owns row l%16 and the 32
 // columns 32·(l/16)… of a chunk, one fully coalesced 1 KiB load per chunk (NVFP4 block scales: one 16-byte load per
 // 8 chunks). What sets the speed is how many of those loads are in flight per CU and how cheaply the activations
-// reach every wave; two kernels:
+// reach every wave; three kernels:
 //  * gemv_row (M <= 2): a workgroup per tile, its waves splitting K into slices of KW = 4/8/16 chunks; each wave
 //    issues its activation slice, the slice's scales and all KW weight chunks at once, stages the activations in its
 //    own LDS region, and computes on the VALU: NVFP4 → BF16 pairs with v_cvt_scalef32_pk_bf16_fp4 (e2m1 × the power-
@@ -18,7 +18,9 @@
 //    gemv_rowp is the same wave layout looping over several tiles per workgroup, for a fused input norm over many
 //    tiles: the norm's statistic (a workgroup barrier on the critical path of every workgroup) is then paid once
 //    per workgroup instead of once per tile.
-//  * gemv_tk (M ≤ 16): MFMA v_mfma_f32_16x16x32_{f16,bf16} with the activations as the A operand (token rows,
+//  * gemv_rowm (2 <= M <= 16): the same wave layout on the matrix cores, the activations of a wave's 512 columns as MFMA
+//    operands in registers for the whole launch (see there).
+//  * gemv_tk (M ≤ 16, where gemv_rowm does not apply): MFMA v_mfma_f32_16x16x32_{f16,bf16} with the activations as the A operand (token rows,
 //    power-of-two prescaled into F16 range: exact above 2^-14 of the row max) and the decoded weights as B (NVFP4 →
 //    exact F16 by v_cvt_scalef32_pk_f16_fp4 and a packed multiply by the mantissa factor). A workgroup stages one K
 //    split of the activations once and streams many tiles against it, so the activations are re-read per workgroup,
@@ -2175,7 +2177,7 @@ Plan plan_tk(const mi_gemv_desc* d, int fmt, int chunks, int n_tiles, int groups
   return best;
 }
 
-// gemv_rowm (3 <= M <= 16, NVFP4 / FP8 / INT4): waves of 512 columns over K splits of at most 12 waves; as many
+// gemv_rowm (2 <= M <= 16): waves of 512 columns over K splits of at most 12 waves; as many
 // workgroups as are resident at once, each over rt tiles
 template <int FMT> __global__ void gemv_rowm(Args a);
 int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
