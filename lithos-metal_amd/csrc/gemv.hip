@@ -1168,10 +1168,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
 #pragma unroll
     for (int s = 0; s < SPC; ++s)
       if (!BA || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
-  float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};       // the lane's output tokens are 4g + i: their 2^p
+  int ps[4] = {0, 0, 0, 0};                     // the lane's output tokens are 4g + i: their p (INT4: of the codes' 2^-24 too)
 #pragma unroll 1
   for (int grp = 0; !BA && grp < ng; ++grp) {
-    float psr[4];
+    int psr[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const uint32_t vv[4] = {xr[r].x, xr[r].y, xr[r].z, xr[r].w};   // past the slice: its last columns again, unused
@@ -1180,9 +1180,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu));
       const uint32_t mx = wave_max_u32(max((uint32_t)m2.x, (uint32_t)m2.y));
-      const int pe = mx == 0 ? 0 : (int)(mx >> 7) - 127 - 14;
+      // not below -126, which FP32 still holds (a smaller maximum ends under 2^14, where F16 holds it as well)
+      const int pe = mx == 0 ? 0 : max((int)(mx >> 7) - 127 - 14, -126);
       const float inv = __uint_as_float((uint32_t)(127 - pe) << 23);
-      psr[r] = __uint_as_float((uint32_t)(127 + pe) << 23);
+      psr[r] = I4 ? pe + 24 : pe;
       f16_t h[8];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -1287,8 +1288,8 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     }
     float* rp = red + wave * a.row_ld + jt * 256;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : acc[i] * (I4 ? ps[i] * 0x1p24f : ps[i])) : 0.0f;
+    for (int i = 0; i < 4; ++i)                 // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
+      rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
   };
   if constexpr (DEPTH == 1) {
     for (int j = 0; j < ntl; ++j) {
@@ -1509,7 +1510,7 @@ __global__ __launch_bounds__(512) void gemv_tk(Args a) {
     } else if constexpr (MF) {
       // F16 operands: 2^-p brings the row max into [2^14, 2^15) (exact for everything within 2^28 of the max)
       mx = wave_max(mx);
-      const int p = mx == 0.0f ? 0 : (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127 - 14;
+      const int p = mx == 0.0f ? 0 : max((int)((__float_as_uint(mx) >> 23) & 0xFF) - 127 - 14, -126);
       const float inv = __uint_as_float((uint32_t)(127 - p) << 23);
       if (lane == 0) pscale[j] = __uint_as_float((uint32_t)(127 + p) << 23);
       wave_lds_sync();

@@ -69,6 +69,17 @@ def test_dequant_every_scale_code(torch_gpu, rng):
     assert np.array_equal(got.view(np.uint32), OF.nvfp4_dequantize(m).view(np.uint32))
 
 
+def _plan(w, x, **kw):
+    """The launch plan (``mi_gemv_plan``) of this GEMV."""
+    import ctypes as C
+    from monolith_mi355 import kernels
+    from monolith_mi355.runtime import hip
+    d, _ = kernels._gemv_desc(w, x, **kw)
+    out = (C.c_int32 * 7)()
+    hip.call("mi_gemv_plan", C.byref(d), out)
+    return list(out)
+
+
 def _run(torch, m, x, **kw):
     """FP32 output, as the reference's gemv_T test reads it (tests/kernels/test_gemv_T.py:21-46)."""
     from monolith_mi355 import kernels
@@ -291,6 +302,48 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
         e = (0, 60)[i == 1] or (0, -60)[i == mtok - 1]
         chk = check_against_oracle(got[i: i + 1] * np.float32(2.0 ** -e), ref[i: i + 1] * np.float32(2.0 ** -e))
         assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
+
+
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
+@pytest.mark.parametrize("mtok", [2, 3, 8])
+@pytest.mark.parametrize("high", [False, True])
+def test_gemv_rowm_extreme_rows(torch_gpu, fmt, mtok, high, rng):
+    """Rows at the ends of the BF16 range keep their values on the matrix cores: one scaled by 2^120 (INT4's 2^24 on top
+    of the row's power is past FP32 from 2^118 on; NVFP4 and FP8 by 2^112: the sum of their unscaled codes has to stay in
+    FP32) or by 2^-120 (below 2^-112 the prescale's own exponent is past it), one of zeros but for a
+    subnormal, beside ordinary ones. The scaled row inside the leaf gate; the subnormal one, whose products FP32 holds only
+    as subnormals, within its smallest normal number."""
+    from monolith_mi355 import kernels
+    torch = torch_gpu
+    k = 3072
+    exp = -120 if not high else 112 if fmt in ("nvfp4", "fp8_e4m3") else 120
+    block = _matrix(fmt, 96, k, rng)
+    per_row = {"nvfp4": 1728, "int4_affine": 1728, "fp8_e4m3": 3072, "bf16": 6144}[fmt]
+    # two tokens: enough rows (the block again and again) for gemv_rowm
+    rep = 1 if mtok > 2 else -(-((40 if fmt == "fp8_e4m3" else 20) << 20) // (per_row * 96)) + 1
+    m = {kk: (np.tile(v, (rep, 1)) if isinstance(v, np.ndarray) and v.ndim == 2 else v) for kk, v in block.items()}
+    w = _upload(torch, m)
+    x = rbf(rng.standard_normal((mtok, k)).astype(np.float32))
+    x[1] *= np.float32(2.0 ** exp)
+    x[1] = rbf(x[1])
+    x[0, :512] = 0.0
+    x[0, 100] = np.float32(2.0 ** -130)
+    only = np.zeros_like(x)
+    only[:, 0] = x[:, 0]
+    only[0, 0], only[0, 700] = 0.0, np.float32(2.0 ** -130)
+    for xi in (x, only):
+        xd = to_dev_bf16(torch, xi)
+        assert _plan(w, xd)[0] == 3
+        got = kernels.gemv(w, xd, out_f32=True).cpu().numpy()
+        assert np.count_nonzero(~np.isfinite(got)) == 0
+        ref = np.tile(ON.matmul_acc(xi.astype(np.float64), _dequant(block).astype(np.float64)), (1, rep))
+        if xi is only:
+            assert np.abs(got[0].astype(np.float64) - ref[0]).max() <= 2.0 ** -126
+            continue
+        for i in range(mtok):
+            e = exp if i == 1 else 0
+            chk = check_against_oracle((got[i: i + 1] * 2.0 ** -e).astype(np.float32), (ref[i: i + 1] * 2.0 ** -e).astype(np.float32))
+            assert chk.ok() and chk.within, (fmt, mtok, high, i, chk)
 
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
