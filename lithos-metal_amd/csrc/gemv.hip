@@ -2178,8 +2178,8 @@ Plan plan_tk(const mi_gemv_desc* d, int fmt, int chunks, int n_tiles, int groups
   return best;
 }
 
-// gemv_rowm (2 <= M <= 16): waves of 512 columns over K splits of at most 12 waves; as many
-// workgroups as are resident at once, each over rt tiles
+// gemv_rowm (2 <= M <= 16): waves of 512 columns over K splits of at most 12 waves; about six waves of workgroups per CU
+// (see below), each over rt tiles
 template <int FMT> __global__ void gemv_rowm(Args a);
 int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
   static std::mutex mu;
@@ -2239,6 +2239,20 @@ Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   const long long slots = std::max<long long>(1, (long long)cu_count() * per_cu_want / ks);
   // every slot takes tiles (strided), so no CU idles for the rounding of tiles per workgroup
   int G = (int)std::min<long long>(n_tiles, slots);
+  // A matrix with more tiles than LDS holds partials of at one workgroup a slot takes whole rounds of workgroups (nothing
+  // needs them resident together). Short slices (up to four waves a workgroup) fill the CU's wave slots in each round, so
+  // that one's conversion hides behind another's stream: NVFP4 248320 x 2048 at M = 3 / 8 / 16 two rounds of one workgroup
+  // a CU 56.5 / 64.1 / 78.4 us, of three 47.4 / 52.4 / 61.2 (gemv_tk 56.0 / 58.6 / 66.0, with partials); longer ones
+  // 151936 x 2560 two rounds of one 44.6 / 50.4 / 62.4, of two 48.8 / 56.3 / 71.7 (gemv_tk 53.9 / 55.7 / 59.2). FP8 has no
+  // other kernel. INT4 and BF16 stay on gemv_tk there: INT4 248320 x 2048 at M = 8 64.7 us against 88.6 here, 128256 x
+  // 3072 53.1 against 57.2, BF16 248320 x 5120 379 against 394.
+  const long long most = (long long)(kMaxLds - fixed) / (S * 1024LL);
+  if (n_tiles > G * most) {
+    if (d->format == FMT_INT4 || d->format == FMT_BF16) return best;
+    const int res = S <= 4 ? std::max(per_cu, 1) : 1;
+    const long long slot = std::max<long long>(1, (long long)cu_count() * res / ks), hold = slot * (most / res);
+    G = (int)std::min<long long>(n_tiles, slot * ((n_tiles + hold - 1) / hold));
+  }
   if (force_rt) G = (n_tiles + force_rt - 1) / force_rt;
   const int rt = (n_tiles + G - 1) / G;
   const size_t lds = fixed + S * region(rt);

@@ -74,6 +74,22 @@ def test_gemv_plans_fit_the_hardware(n, k, m):
     assert (ws > 0) == (ks > 1)
 
 
+@pytest.mark.parametrize("fmt,k", [("fp8_e4m3", 64), ("fp8_e4m3", 1536), ("fp8_e4m3", 2048), ("fp8_e4m3", 2560),
+                                   ("fp8_e4m3", 3072), ("fp8_e4m3", 5120), ("fp8_e4m3", 17408), ("nvfp4", 512),
+                                   ("nvfp4", 2048), ("nvfp4", 2560), ("nvfp4", 3072), ("nvfp4", 6144), ("nvfp4", 17408)])
+def test_gemv_rowm_plans_cover_any_height(fmt, k):
+    """gemv_rowm has a plan for every row count (a vocabulary-sized head among them), whose workgroups cover every tile
+    with partials that fit LDS: FP8 has no other kernel at M >= 3."""
+    from monolith_mi355.runtime import hip
+    out = (C.c_int32 * 7)()
+    for m in (3, 8, 16):
+        for n in (16, 4096, 34816, 111000, 128256, 131072, 135000, 151936, 168000, 201088, 248320, 262144, 1 << 20):
+            hip.call("mi_gemv_plan", C.byref(_desc(hip, format=hip.MI_FMT[fmt], n=n, k=k, m=m, ldx=k, ldy=n)), out)
+            kernel, waves, kw, rt, ks, lds, wgs = list(out)
+            assert kernel == 3 and lds <= 160 * 1024 and waves <= 12, (m, n, list(out))
+            assert rt * (wgs // ks) >= -(-n // 16) and wgs % ks == 0, (m, n, list(out))
+
+
 def test_gemv_rejects_bad_descriptors_before_launch():
     from monolith_mi355.runtime import hip
     lib = hip.load()

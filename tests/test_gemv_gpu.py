@@ -304,6 +304,33 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
         assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
 
 
+@pytest.mark.parametrize("fmt,n,k", [("fp8_e4m3", 170056, 2048), ("nvfp4", 170056, 2048), ("fp8_e4m3", 57352, 6144)])
+def test_gemv_rowm_tall(torch_gpu, fmt, n, k):
+    """A matrix of more tiles than one round of workgroups holds partials of (the last tile half full): every row of
+    the product against the decoded matrix in float64. The packed bytes are random (any are codes of the format; the
+    decode itself is pinned elsewhere)."""
+    from monolith_mi355 import kernels
+    from monolith_mi355.formats.pack import pack_bytes
+    torch = torch_gpu
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    data = torch.randint(0, 256, (pack_bytes(fmt, n, k),), dtype=torch.uint8, generator=g, device="cuda")
+    data &= 0xF7 if fmt == "fp8_e4m3" else 0x7F                          # no NaN code / NVFP4 scale
+    if fmt == "nvfp4":
+        data &= 0xBF                                                     # scales below 2
+    w = kernels.PackedWeight(fmt, n, k, 1, data, torch.rand((n + 15) // 16 * 16, generator=g, device="cuda"))
+    x = torch.randn(5, k, generator=g, device="cuda").to(torch.bfloat16)
+    plan = _plan(w, x)
+    assert plan[0] == 3 and plan[3] * plan[1] * 1024 <= 160 * 1024 and plan[6] > 256, plan
+    got = kernels.gemv(w, x, out_f32=True)
+    wd = kernels.dequant(w)
+    for lo in range(0, n, 32768):
+        part = wd[lo: lo + 32768].double()
+        ref = x.double() @ part.T
+        bound = x.double().abs() @ part.abs().T          # 32-bit sums of k products: a part of sum |x·w|
+        assert ((got[:, lo: lo + 32768].double() - ref).abs() <= 2.0 ** -18 * bound).all(), (fmt, lo)
+
+
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("mtok", [2, 3, 8])
 @pytest.mark.parametrize("high", [False, True])
