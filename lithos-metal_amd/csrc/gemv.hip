@@ -1061,7 +1061,8 @@ void gemv_rowp(Args a) {
 // every one of them. The
 // wave's activations for those chunks stay in VGPRs for the whole launch as the F16 A operands of
 // v_mfma_f32_16x16x32_f16 (token = A row; each token power-of-two scaled into F16 range over the wave's slice;
-// a fused input norm runs as its own launch before, see wants_prenorm); the weights are the B operand, decoded exactly to F16. Each wave
+// a fused input norm runs as its own launch before, see wants_prenorm; TWO, the instantiation for M = 2, takes it itself);
+// the weights are the B operand, decoded exactly to F16. Each wave
 // keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5;
 // BF16 one, its tile is 16 chunks) and issues the next as soon
 // as one is consumed. FP8 and BF16 take BF16 operands instead (their weights
@@ -1070,10 +1071,11 @@ void gemv_rowp(Args a) {
 // tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to exact F16
 // integers, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
 // scaled and offset by its (scale, bias) pair with the token's Σx over the group (held per lane for the launch).
-// LDS: (INT4: Σx [S][KW][2][16]) | red [S][row_ld floats]: a wave's activation stage, then its [rt][16 tokens][16 rows].
+// LDS: (TWO: Σx² [2][12]) | (INT4: Σx [S][KW][2][16]) | red [S][row_ld floats]: a wave's activation stage, then its [rt][16 tokens][16 rows].
 constexpr int ROWM_SLD = 1024 + 16;             // bytes of a staged activation row (512 columns), padded
+constexpr int ROWM_S = 12;                      // waves at most
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
-template <int FMT>
+template <int FMT, bool TWO>
 __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   constexpr int KC = chunk_cols(FMT), KW = 512 / KC;   // a wave's slice is 512 columns: 4 NVFP4 / INT4, 8 FP8, 16 BF16 chunks
   constexpr int SPC = KC / 32;                  // MFMA steps per chunk: the lane's KC/4 columns, 8 per step
@@ -1095,7 +1097,8 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   const int g = lane >> 4, m_row = lane & 15;
   const uint8_t* wmat = a.w;
   auto tile_of = [&](int j) { return (int)blockIdx.x + j * G; };
-  float* sxl = reinterpret_cast<float*>(smem);                                  // INT4: [S][KW][2][16]
+  float* stat = reinterpret_cast<float*>(smem);                                 // TWO: [2][ROWM_S]
+  float* sxl = stat + (TWO ? 2 * ROWM_S : 0);                                  // INT4: [S][KW][2][16]
   float* red = sxl + (I4 ? S * KW * 2 * 16 : 0);                               // [S][row_ld]: per wave its activation
                                                                                // stage, then its tiles' [rt][16][16]
 
@@ -1116,8 +1119,44 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] = *reinterpret_cast<const uint4*>(xbase + (long long)min(4 * grp + r, cnt - 1) * a.ldx);
   };
+  // one row's slice into the stage, as F16 by the row's power; the power p
+  auto stage_row = [&](int r, const uint32_t (&vv)[4]) {               // past the slice: its last columns again, unused
+    // the max on the BF16 magnitudes as integers (the same order for finite values)
+    u16x2_t m2 = {0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu));
+    const uint32_t mx = wave_max_u32(max((uint32_t)m2.x, (uint32_t)m2.y));
+    // not below -126, which FP32 still holds (a smaller maximum ends under 2^14, where F16 holds it as well)
+    const int pe = mx == 0 ? 0 : max((int)(mx >> 7) - 127 - 14, -126);
+    const float inv = __uint_as_float((uint32_t)(127 - pe) << 23);
+    f16_t h[8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      h[2 * q] = (f16_t)(bf16_bits_to_f32(vv[q] & 0xFFFFu) * inv);
+      h[2 * q + 1] = (f16_t)(bf16_bits_to_f32(vv[q] >> 16) * inv);
+    }
+    f16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns,
+    if constexpr (I4) {                                                // 1/16 where the code comes as 16n (exact
+#pragma unroll                                                         // above 2^-10 of a row whose max is 2^14)
+      for (int e = 0; e < 8; ++e)
+        if (int4_high(e)) o[e] *= (f16_t)0.0625f;
+    }
+    *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
+    return I4 ? pe + 24 : pe;
+  };
   uint4 xr[4], xn[4], xa[KW][SPC];
-  if constexpr (BA) {
+  float4 w0, w1;
+  if constexpr (TWO) {
+    xr[0] = *reinterpret_cast<const uint4*>(xbase);
+    xr[1] = *reinterpret_cast<const uint4*>(xbase + a.ldx);
+    if (a.norm_w) {
+      const float* nw = a.norm_w + c0 * KC + min(8 * lane, cols - 8);
+      w0 = *reinterpret_cast<const float4*>(nw);
+      w1 = *reinterpret_cast<const float4*>(nw + 4);
+    }
+  } else if constexpr (BA) {
     const uint16_t* xrow = a.x + (long long)min(m_row, cnt - 1) * a.ldx + c0 * KC;
 #pragma unroll
     for (int cc = 0; cc < KW; ++cc)
@@ -1167,55 +1206,61 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   for (int cc = 0; cc < KW; ++cc)               // padding tokens: zero operands
 #pragma unroll
     for (int s = 0; s < SPC; ++s)
-      if (!BA || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
+      if (TWO || !BA || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
   int ps[4] = {0, 0, 0, 0};                     // the lane's output tokens are 4g + i: their p (INT4: of the codes' 2^-24 too)
+  auto take_rows = [&] {                        // the lane's token from the stage
+#pragma unroll
+    for (int cc = 0; cc < KW; ++cc)
+#pragma unroll
+      for (int s = 0; s < SPC; ++s)
+        xa[cc][s] = *reinterpret_cast<const uint4*>(stage + (m_row & 3) * ROWM_SLD + 2 * (cc * KC + xcol(s)));
+  };
+  if constexpr (TWO) {
+    // Two tokens: the fused norm here (one row load, one barrier among the waves), so the call stays one launch without
+    // scratch. A wave's slice is one slice of the statistic, its order and the values those of norm_apply, bit for bit.
+    uint32_t v[2][4] = {{xr[0].x, xr[0].y, xr[0].z, xr[0].w}, {xr[1].x, xr[1].y, xr[1].z, xr[1].w}};
+    if (a.norm_w) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const float sv = vec_sumsq(v[t]), sq = wave_sum(8 * lane < cols ? sv : 0.0f);
+        if (lane == 0) stat[t * ROWM_S + wave] = sq;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float ssq = 0.0f;
+        for (int i = 0; i < S; ++i) ssq += stat[t * ROWM_S + i];
+        norm_vec(v[t], 1.0f / sqrtf(ssq / (float)a.k + a.eps), w0, w1, v[t]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if constexpr (BA) *reinterpret_cast<uint4*>(stage + t * ROWM_SLD + 16 * lane) = uint4{v[t][0], v[t][1], v[t][2], v[t][3]};
+      else ps[t] = stage_row(t, v[t]);          // in every lane; the k-group 0 lanes hold the two tokens' outputs
+    }
+    wave_lds_sync();
+    if (m_row < 2) take_rows();
+    wave_lds_sync();
+  } else {
 #pragma unroll 1
-  for (int grp = 0; !BA && grp < ng; ++grp) {
-    int psr[4];
+    for (int grp = 0; !BA && grp < ng; ++grp) {
+      int psr[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint32_t vv[4] = {xr[r].x, xr[r].y, xr[r].z, xr[r].w};   // past the slice: its last columns again, unused
-      // the max on the BF16 magnitudes as integers (the same order for finite values)
-      u16x2_t m2 = {0, 0};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu));
-      const uint32_t mx = wave_max_u32(max((uint32_t)m2.x, (uint32_t)m2.y));
-      // not below -126, which FP32 still holds (a smaller maximum ends under 2^14, where F16 holds it as well)
-      const int pe = mx == 0 ? 0 : max((int)(mx >> 7) - 127 - 14, -126);
-      const float inv = __uint_as_float((uint32_t)(127 - pe) << 23);
-      psr[r] = I4 ? pe + 24 : pe;
-      f16_t h[8];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        h[2 * q] = (f16_t)(bf16_bits_to_f32(vv[q] & 0xFFFFu) * inv);
-        h[2 * q + 1] = (f16_t)(bf16_bits_to_f32(vv[q] >> 16) * inv);
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t vv[4] = {xr[r].x, xr[r].y, xr[r].z, xr[r].w};
+        psr[r] = stage_row(r, vv);
       }
-      f16x8 o;
+      wave_lds_sync();
+      if (g == grp) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns,
-      if constexpr (I4) {                                                // 1/16 where the code comes as 16n (exact
-#pragma unroll                                                          // above 2^-10 of a row whose max is 2^14)
-        for (int e = 0; e < 8; ++e)
-          if (int4_high(e)) o[e] *= (f16_t)0.0625f;
+        for (int r = 0; r < 4; ++r) ps[r] = psr[r];
       }
-      *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
+      if ((m_row >> 2) == grp && m_row < cnt) take_rows();
+      wave_lds_sync();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) xr[r] = xn[r];
+      if (grp + 2 < ng) load4(xn, grp + 2);
     }
-    wave_lds_sync();
-    if (g == grp) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ps[r] = psr[r];
-    }
-    if ((m_row >> 2) == grp && m_row < cnt) {
-#pragma unroll
-      for (int cc = 0; cc < KW; ++cc)
-#pragma unroll
-        for (int s = 0; s < SPC; ++s)
-          xa[cc][s] = *reinterpret_cast<const uint4*>(stage + (m_row & 3) * ROWM_SLD + 2 * (cc * KC + xcol(s)));
-    }
-    wave_lds_sync();
-#pragma unroll
-    for (int r = 0; r < 4; ++r) xr[r] = xn[r];
-    if (grp + 2 < ng) load4(xn, grp + 2);
   }
   // INT4: Σx (prescaled F16) per 64-column group — steps {0, 1} and {2, 3} of each chunk — per token (the sum over
   // its four k-group lanes), kept in the wave's LDS rows: tile_mma reads those of its output tokens 4g + i
@@ -1288,8 +1333,8 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     }
     float* rp = red + wave * a.row_ld + jt * 256;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)                 // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
-      rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
+    for (int i = 0; i < (TWO ? 2 : 4); ++i)     // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
+      if (!TWO || g == 0) rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
   };
   if constexpr (DEPTH == 1) {
     for (int j = 0; j < ntl; ++j) {
@@ -2180,24 +2225,24 @@ Plan plan_tk(const mi_gemv_desc* d, int fmt, int chunks, int n_tiles, int groups
 
 // gemv_rowm (2 <= M <= 16): waves of 512 columns over K splits of at most 12 waves; about six waves of workgroups per CU
 // (see below), each over rt tiles
-template <int FMT> __global__ void gemv_rowm(Args a);
-int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
+template <int FMT, bool TWO> __global__ void gemv_rowm(Args a);
+int rowm_blocks_per_cu(int fmt, bool two, int threads, size_t lds) {
   static std::mutex mu;
   static std::map<std::tuple<int, size_t, int>, int> cache;
   int dev = 0;
   (void)hipGetDevice(&dev);
   (void)hipGetLastError();
-  const auto key = std::make_tuple(threads * 8 + fmt, lds, dev);
+  const auto key = std::make_tuple((threads * 8 + fmt) * 2 + two, lds, dev);
   {
     std::lock_guard<std::mutex> lk(mu);
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
   }
   int n = 0;
-  const void* kern = fmt == FMT_FP8    ? reinterpret_cast<const void*>(gemv_rowm<FMT_FP8>)
-                     : fmt == FMT_BF16 ? reinterpret_cast<const void*>(gemv_rowm<FMT_BF16>)
-                     : fmt == FMT_INT4 ? reinterpret_cast<const void*>(gemv_rowm<FMT_INT4>)
-                                       : reinterpret_cast<const void*>(gemv_rowm<FMT_NVFP4>);
+  const void* kern = nullptr;
+#define MI_ROWM_K(F) if (fmt == F) kern = two ? reinterpret_cast<const void*>(gemv_rowm<F, true>) : reinterpret_cast<const void*>(gemv_rowm<F, false>);
+  MI_ROWM_K(FMT_NVFP4) MI_ROWM_K(FMT_INT4) MI_ROWM_K(FMT_BF16) MI_ROWM_K(FMT_FP8)
+#undef MI_ROWM_K
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, threads, lds) !=
           hipSuccess || n <= 0) {
     (void)hipGetLastError();
@@ -2210,8 +2255,8 @@ int rowm_blocks_per_cu(int fmt, int threads, size_t lds) {
 
 Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   Plan best{};
-  if (d->groups || d->gnorm_w || d->norm_w ||
-      d->m < 2 || d->m > 16 ||
+  const bool two = d->m == 2;                     // its own instantiation, which fuses the input norm
+  if (d->groups || d->gnorm_w || (d->norm_w && !two) || d->m < 2 || d->m > 16 ||
       (d->format == FMT_NVFP4 && chunks < 4))     // less than a slice of K: one short stream a tile, gemv_tk's
     return best;
   const int kw = 512 / chunk_cols(d->format);    // chunks per wave (512 columns)
@@ -2226,10 +2271,11 @@ Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   if (ks > 1) kc = (kc + 7) / 8 * 8;             // splits on scale-group boundaries (whole waves for FP8)
   if (kc > 12 * kw || (ks > 1 && (ks - 1) * kc >= chunks)) return best;
   const int S = (kc + kw - 1) / kw;
-  const size_t fixed = d->format == FMT_INT4 ? (size_t)S * (512 / chunk_cols(FMT_INT4)) * 2 * 16 * 4 : 0;
+  const size_t fixed = (two ? 2 * ROWM_S * sizeof(float) : 0) +
+                       (d->format == FMT_INT4 ? (size_t)S * (512 / chunk_cols(FMT_INT4)) * 2 * 16 * 4 : 0);
   // a wave's LDS region: its activation stage (4 rows), then a 1 KiB partial per tile
   auto region = [](int rt) { return std::max<size_t>(4 * ROWM_SLD, (size_t)rt * 1024); };
-  const int per_cu = rowm_blocks_per_cu(d->format, 64 * S, fixed + S * region(4));
+  const int per_cu = rowm_blocks_per_cu(d->format, two, 64 * S, fixed + S * region(4));
   // Workgroups per CU: as many as make six waves, at least one. The activations are converted once per workgroup, on
   // every CU the same work for each resident workgroup, so fewer workgroups over more tiles win as long as a CU has
   // about four waves' loads in flight (one workgroup of 6 waves a CU over 6 tiles instead of two over 3, N = 24576,
@@ -2277,22 +2323,22 @@ size_t fold_counter_bytes(int) { return kFoldCounterBytes; }
 // behind a workgroup barrier. Measured on the 27B shapes at M = 8, bit-identical: gate|up 33.0 → 30.5 µs, in_proj
 // 24.7 → 22.0 µs (the extra launch ≈ 2.9 µs). Inside gemv_rowm's staging of four rows at a time (statistic through LDS,
 // one barrier a group) it still measured 2 to 4 us a group more than the launch: gate|up at M = 3 / 8 / 16 23.5 / 23.8 /
-// 27.7 us with the launch, 27.0 / 31.4 / 39.4 fused. At M <= 2 gemv_row's fused norm costs less than a launch.
+// 27.7 us with the launch, 27.0 / 31.4 / 39.4 fused. At M <= 2 the norm is fused in gemv_row and in gemv_rowm's two-token
+// instantiation, which takes no scratch with it: graphs captured on one stream and threads that share one stay apart.
 bool wants_prenorm(const mi_gemv_desc* d) {
   const int rows = d->groups ? std::min(16, d->m) : d->m;
   return d->norm_w && rows > 2 && !(d->groups && d->x_per_slot) && !d->route_logits && d->k % 8 == 0;
 }
 
 // Two tokens over a large weight stream run on gemv_rowm: gemv_row's dot products for two tokens (VALU) fall behind the
-// stream, the matrix cores take any M at the price of one, and the norm's launch costs less than normalizing two rows
-// in every workgroup. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 42.9 → 23.3 us, without 29.0 →
-// 20.7, in_proj with the norm 23.4 → 15.5, INT4 gate|up 29.8 → 21.6, FP8 in_proj 31.2 → 20.5, q|k|v (20.6
-// MB, norm) 11.5 → 10.8, BF16 8192 x 4096 17.5 → 13.5. Below, and for a short K (few waves share a workgroup's
-// activations), gemv_row wins or ties: N = 34816 with the norm K = 1024 / 1536 / 2048 / 3072 9.8 / 12.7 / 14.3 / 24.4 against
-// 10.6 / 12.5 / 13.3 / 16.8 us, without it 7.9 / 9.3 / 10.7 / 16.6 against 8.3 / 9.9 / 10.9 / 14.1, INT4 K = 2048 16.0
-// against 18.2, FP8 8192 x 4096 (33.6 MB, norm) 10.7 against 10.9, BF16 12288 x 2048 13.4 against 13.1, FP8 4096 x 4096
-// (16.8 MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4. A K that gemv_rowm would split (over 6144) stays on
-// gemv_row, which folds its splits in the kernel and needs no partials for them.
+// stream and normalize both rows in every tile's workgroup; the matrix cores take any M at the price of one, the norm is
+// taken once for a workgroup's tiles. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 41.8 → 21.4 us,
+// without 28.8 → 20.3, in_proj with the norm 23.5 → 14.3, INT4 gate|up 30.1 → 20.6, with the norm 46.0 → 23.0, FP8
+// in_proj 31.3 → 17.4, NVFP4 248320 x 5120 with the norm 248 → 124, BF16 8192 x 4096 17.5 → 12.9. Below, and for a short K
+// (few waves share a workgroup's activations), gemv_row won or tied: without the norm N = 34816, K = 1024 / 1536 / 2048 /
+// 3072 7.9 / 9.3 / 10.7 / 16.6 against 8.3 / 9.9 / 10.9 / 14.1 us, INT4 K = 2048 16.0 against 18.2, FP8 4096 x 4096 (16.8
+// MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4. A K that gemv_rowm would split (over 6144) stays on gemv_row,
+// which folds its splits in the kernel and needs no partials for them.
 constexpr size_t kRowmTwoBytes = 20u << 20;
 bool rowm_at_two(const mi_gemv_desc* d) {
   const size_t least = d->format == FMT_FP8 ? 2 * kRowmTwoBytes : kRowmTwoBytes;
@@ -2301,13 +2347,9 @@ bool rowm_at_two(const mi_gemv_desc* d) {
          !getenv("MI_GEMV_KERNEL") && !getenv("MI_GEMV_ROW");
 }
 
-// two: whether two tokens may take gemv_rowm, which needs scratch where gemv_row does not
-Plan make_plan(const mi_gemv_desc* d, bool two = true) {
-  if (two && rowm_at_two(d)) {
-    mi_gemv_desc plain = *d;
-    plain.norm_w = nullptr;
-    Plan p = plan_rowm(&plain, d->k / chunk_cols(d->format), (d->n + 15) / 16);
-    p.prenorm = p.kernel != 0 && d->norm_w;
+Plan make_plan(const mi_gemv_desc* d) {
+  if (rowm_at_two(d)) {
+    const Plan p = plan_rowm(d, d->k / chunk_cols(d->format), (d->n + 15) / 16);
     if (p.kernel && p.ks == 1) return p;
   }
   if (d->conv_w) {                              // the conv epilogue lives in gemv_row: one tile per workgroup
@@ -2441,8 +2483,9 @@ void launch_reduce(const Args& a, hipStream_t s) {
 template <int FMT>
 void launch(const Args& a, const Plan& p, int groups, hipStream_t s) {
   if (p.kernel == 3) {
-    allow_lds(gemv_rowm<FMT>);
-    hipLaunchKernelGGL(gemv_rowm<FMT>, dim3(p.G, 1, p.ks), dim3(64 * p.S), p.lds_bytes, s, a);
+    const dim3 g(p.G, 1, p.ks);
+    if (a.m == 2) { allow_lds(gemv_rowm<FMT, true>); hipLaunchKernelGGL((gemv_rowm<FMT, true>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
+    else { allow_lds(gemv_rowm<FMT, false>); hipLaunchKernelGGL((gemv_rowm<FMT, false>), g, dim3(64 * p.S), p.lds_bytes, s, a); }
     if (p.ks > 1) launch_reduce(a, s);
     return;
   }
@@ -2500,20 +2543,8 @@ namespace {
 // device-resident array), or null: the caller's workspace, else the library's scratch.
 int gemv_impl(const mi_gemv_desc* d, void* stream, void* fixed_ws, size_t fixed_bytes, const char* name) {
   if (int rc = check_desc(d)) return rc;
-  Plan p = make_plan(d);
+  const Plan p = make_plan(d);
   MI_REQUIRE(p.kernel, "%s: no launch plan fits (k=%d, m=%d)", name, d->k, d->m);
-  // two tokens on gemv_rowm without the scratch it needs (a workspace sized for less, a stream captured before its first
-  // eager call): gemv_row
-  void* unused = nullptr;
-  if (p.kernel == 3 && d->m == 2) {
-    if (const size_t need = workspace_need(d, p)) {
-      const bool ok = fixed_ws ? need <= fixed_bytes
-                      : d->workspace ? d->workspace_bytes >= need
-                                     : mi_library_scratch(MI_SCRATCH_GEMV, need, static_cast<hipStream_t>(stream), &unused) == MI_OK;
-      if (!ok) p = make_plan(d, false);
-      MI_REQUIRE(p.kernel, "%s: no launch plan fits (k=%d, m=%d)", name, d->k, d->m);
-    }
-  }
   MI_REQUIRE(!d->route_logits || (p.kernel == 1 && p.ks == 1), "%s: routing in the launch runs on gemv_row", name);
   Args a{};
   a.w = static_cast<const uint8_t*>(d->w);

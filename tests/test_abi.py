@@ -90,6 +90,26 @@ def test_gemv_rowm_plans_cover_any_height(fmt, k):
             assert rt * (wgs // ks) >= -(-n // 16) and wgs % ks == 0, (m, n, list(out))
 
 
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
+def test_two_tokens_with_a_norm_take_no_scratch(fmt):
+    """One token or two with a fused input norm are one launch without scratch, on either kernel: calls that overlap
+    (graphs captured on one stream, threads that share one) have nothing in common to write."""
+    from monolith_mi355.runtime import hip
+    out, kernels = (C.c_int32 * 7)(), set()
+    for n, k in ((512, 2048), (16480, 5120), (34816, 5120), (12288, 3072), (20480, 6144), (248320, 5120)):
+        for m in (1, 2):
+            d = _desc(hip, format=hip.MI_FMT[fmt], n=n, k=k, m=m, ldx=k, ldy=n, norm_w=256)
+            hip.call("mi_gemv_plan", C.byref(d), out)
+            if out[4] > 1:                                   # K splits (a long K): partials, with or without a norm
+                d.norm_w = 0
+                hip.call("mi_gemv_plan", C.byref(d), out)
+                assert out[4] > 1, (n, k, m)
+                continue
+            kernels.add((m, out[0]))
+            assert hip.load().mi_gemv_workspace_bytes(C.byref(d)) == 0, (n, k, m)
+    assert {(1, 1), (2, 1), (2, 3)} <= kernels
+
+
 def test_gemv_rejects_bad_descriptors_before_launch():
     from monolith_mi355.runtime import hip
     lib = hip.load()

@@ -378,7 +378,7 @@ def test_gemv_rowm_extreme_rows(torch_gpu, fmt, mtok, high, rng):
 @pytest.mark.parametrize("norm", [False, True])
 def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
     """Two tokens on either side of the weight bytes where gemv_rowm takes over (20 MiB, FP8 40): the plan, the rows against the
-    oracle's float64 product, and a workspace too small for gemv_rowm's scratch (then gemv_row, the same gate)."""
+    oracle's float64 product, with a workspace too small for any scratch as well (a plan without splits takes none)."""
     import ctypes as C
     from monolith_mi355 import kernels
     from monolith_mi355.runtime import hip
@@ -407,6 +407,54 @@ def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
         got = kernels.gemv(w, xd, out_f32=True, workspace=ws, **kw).cpu().numpy()
         chk = check_against_oracle(got, ref)
         assert (chk.ok_rounded() if norm else chk.ok()) and chk.within, (fmt, big, norm, chk)
+
+
+@pytest.mark.parametrize("fmt,n,k", [("nvfp4", 12296, 3200), ("nvfp4", 7000, 6144), ("int4_affine", 12296, 3200),
+                                     ("fp8_e4m3", 13720, 3136), ("fp8_e4m3", 170056, 3072), ("bf16", 5320, 2080)])
+def test_gemv_two_tokens_norm_in_one_launch(torch_gpu, fmt, n, k):
+    """Two tokens on gemv_rowm with the input norm fused, over a last slice of one chunk, whole slices up to twelve
+    waves, and more tiles than one round of workgroups: the bits of norm_apply and the plain GEMV after it (at a row
+    stride past K), of mi_gemv_noalloc, and of a graph captured before any eager call on its stream, replayed with
+    eager work between; the plain GEMV's rows against the decoded matrix in float64. The packed bytes are random."""
+    import ctypes as C
+    from monolith_mi355 import kernels
+    from monolith_mi355.formats.pack import pack_bytes
+    from monolith_mi355.runtime import hip
+    torch = torch_gpu
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    data = torch.randint(0, 256, (pack_bytes(fmt, n, k),), dtype=torch.uint8, generator=g, device="cuda")
+    data &= {"fp8_e4m3": 0xF7, "bf16": 0xBF}.get(fmt, 0x3F)      # finite codes, BF16 weights and scales
+    rs = torch.rand((n + 15) // 16 * 16, generator=g, device="cuda") if fmt in ("nvfp4", "fp8_e4m3") else None
+    w = kernels.PackedWeight(fmt, n, k, 1, data, rs)
+    x = torch.randn(2, k + 24, generator=g, device="cuda").to(torch.bfloat16)[:, :k]
+    nw = 1.0 + 0.1 * torch.randn(k, generator=g, device="cuda")
+    kw = dict(norm_w=nw, eps=1e-6, out_f32=True)
+    assert _plan(w, x, **kw)[0] == 3
+    xn = kernels.norm_apply(x, nw, eps=1e-6)
+    want = kernels.gemv(w, xn, out_f32=True)
+    wd = kernels.dequant(w)
+    for lo in range(0, n, 32768):
+        part = wd[lo: lo + 32768].double()
+        bound = xn.double().abs() @ part.abs().T                 # 32-bit sums of k products: a part of sum |x·w|
+        assert ((want[:, lo: lo + 32768].double() - xn.double() @ part.T).abs() <= 2.0 ** -18 * bound).all()
+    assert torch.equal(kernels.gemv(w, x, **kw), want)
+    out = torch.zeros_like(want)
+    d, _ = kernels._gemv_desc(w, x, out=out, **kw)
+    torch.cuda.synchronize()
+    hip.call("mi_gemv_noalloc", C.byref(d), hip.stream_handle())
+    assert torch.equal(out, want)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = hip.Graph(s)
+    with torch.cuda.stream(s), graph:
+        kernels.gemv(w, x, out=out, **kw)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.launch()
+        s.synchronize()
+        assert torch.equal(out, want)
 
 
 def test_fp8_dequant_every_code(torch_gpu):
