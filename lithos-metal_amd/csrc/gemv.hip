@@ -194,18 +194,14 @@ __device__ __forceinline__ f16x8 int4_decode8(uint32_t dw) {
   return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
-// The same codes as F16 denormals, the nibbles where they stand: n·2^-24 (elements 0, 1, 4, 5) or 16n·2^-24 (2, 3, 6,
-// 7: their activations carry the 1/16) — exact, and five instructions for eight weights instead of eleven
+// The same codes as F16 denormals n·2^-24: exact, and seven instructions for eight weights instead of eleven. (Two fewer
+// with the odd nibbles left where they stand, as 16n, cost their activations four binades at the low end.)
 __device__ __forceinline__ f16x8 int4_decode8_denormal(uint32_t dw) {
-  const uint32_t hi = dw >> 8;
   union { uint32_t u[4]; f16x8 h; } p;
-  p.u[0] = dw & 0x000F000Fu;
-  p.u[1] = dw & 0x00F000F0u;
-  p.u[2] = hi & 0x000F000Fu;
-  p.u[3] = hi & 0x00F000F0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p.u[i] = (dw >> (4 * i)) & 0x000F000Fu;
   return p.h;
 }
-__device__ __forceinline__ bool int4_high(int e) { return (e & 2) != 0; }   // the elements that carry 16n
 
 // FP8 E4M3: codes 2j, 2j+1 of a dword (hi: 2, 3) → exact BF16 / F16 pairs (scale 1: the tensor scale is the row's)
 __device__ __forceinline__ bf16x2 cvt_fp8x2_bf16(uint32_t dw, bool hi) {
@@ -1068,9 +1064,9 @@ void gemv_rowp(Args a) {
 // as one is consumed. FP8 and BF16 take BF16 operands instead (their weights
 // are exact BF16, the activations as they are): BF16 8192 x 4096 at M = 3 / 8 / 16 22.3 / 22.5 / 23.2 us on gemv_tk, 13.5 /
 // 14.0 / 14.8 here. A
-// tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to exact F16
-// integers, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
-// scaled and offset by its (scale, bias) pair with the token's Σx over the group (held per lane for the launch).
+// tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to F16
+// denormals n·2^-24, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
+// scaled and offset by its (scale, bias) pair with the token's Σx over the group (in the wave's LDS rows).
 // LDS: (TWO: Σx² [2][12]) | (INT4: Σx [S][KW][2][16]) | red [S][row_ld floats]: a wave's activation stage, then its [rt][16 tokens][16 rows].
 constexpr int ROWM_SLD = 1024 + 16;             // bytes of a staged activation row (512 columns), padded
 constexpr int ROWM_S = 12;                      // waves at most
@@ -1137,12 +1133,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     }
     f16x8 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns,
-    if constexpr (I4) {                                                // 1/16 where the code comes as 16n (exact
-#pragma unroll                                                         // above 2^-10 of a row whose max is 2^14)
-      for (int e = 0; e < 8; ++e)
-        if (int4_high(e)) o[e] *= (f16_t)0.0625f;
-    }
+    for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns
     *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
     return I4 ? pe + 24 : pe;
   };
@@ -1275,7 +1266,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         for (int s = 2 * gp; s < 2 * gp + 2; ++s) {
           const f16x8 h = __builtin_bit_cast(f16x8, xa[cc][s]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) sx += (float)h[e] * (int4_high(e) ? 16.0f : 1.0f);
+          for (int e = 0; e < 8; ++e) sx += (float)h[e];
         }
         sx = add_xor32(add_xor16(cc < kw ? sx : 0.0f));
         if (g == 0) sxw[(cc * 2 + gp) * 16 + m_row] = sx * 0x1p-24f;     // in the units of the codes' dot products

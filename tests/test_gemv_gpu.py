@@ -333,6 +333,40 @@ def test_gemv_rowm_tall(torch_gpu, fmt, n, k):
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("mtok", [2, 3, 8])
+def test_gemv_rowm_small_beside_large(torch_gpu, fmt, mtok, rng):
+    """One value of a 512-column slice 2^30 above the others, on a zero weight: the small ones keep all their bits (eight,
+    with F16's 24 below the slice's maximum), so the rest of the sum is a 32-bit sum."""
+    _small_beside_large(torch_gpu, fmt, mtok, (-30,), rng)
+
+
+def _small_beside_large(torch, fmt, mtok, exps, rng):
+    from monolith_mi355 import kernels
+    k, big = 3072, 1000
+    block = _matrix(fmt, 96, k, rng)
+    block["weight"][:, big // 2 if fmt in ("nvfp4", "int4_affine") else big] = 0
+    if fmt == "int4_affine":                                  # code 0 without an offset in its group
+        block["biases"][:, big // 64] = 0
+    wd = _dequant(block).astype(np.float64)
+    assert not wd[:, big].any()
+    per_row = {"nvfp4": 1728, "int4_affine": 1728, "fp8_e4m3": 3072, "bf16": 6144}[fmt]
+    rep = 1 if mtok > 2 else -(-((40 if fmt == "fp8_e4m3" else 20) << 20) // (per_row * 96)) + 1
+    m = {kk: (np.tile(v, (rep, 1)) if isinstance(v, np.ndarray) and v.ndim == 2 else v) for kk, v in block.items()}
+    w = _upload(torch, m)
+    for exp in exps:
+        x = rbf((1 + rng.random((mtok, k))) * np.where(rng.random((mtok, k)) < 0.5, -1, 1))
+        up = min(0, -110 - exp)                               # the small ones stay above 2^-110
+        x = rbf(x * np.float32(2.0 ** (exp - up)))
+        x[:, big] = rbf(np.float32(1.5 * 2.0 ** -up))
+        xd = to_dev_bf16(torch, x)
+        assert _plan(w, xd)[0] == 3
+        got = kernels.gemv(w, xd, out_f32=True).cpu().numpy().astype(np.float64)
+        ref = np.tile(x.astype(np.float64) @ wd.T, (1, rep))
+        bound = np.tile(np.abs(x.astype(np.float64)) @ np.abs(wd).T, (1, rep))
+        assert (np.abs(got - ref) <= 2.0 ** -18 * bound).all(), (fmt, mtok, exp)
+
+
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
+@pytest.mark.parametrize("mtok", [2, 3, 8])
 @pytest.mark.parametrize("high", [False, True])
 def test_gemv_rowm_extreme_rows(torch_gpu, fmt, mtok, high, rng):
     """Rows at the ends of the BF16 range keep their values on the matrix cores: one scaled by 2^120 (INT4's 2^24 on top
