@@ -1057,7 +1057,8 @@ void gemv_rowp(Args a) {
 // every one of them. The
 // wave's activations for those chunks stay in VGPRs for the whole launch as the F16 A operands of
 // v_mfma_f32_16x16x32_f16 (token = A row; each token power-of-two scaled into F16 range over the wave's slice;
-// a fused input norm runs as its own launch before, see wants_prenorm; TWO, the instantiation for M = 2, takes it itself);
+// a fused input norm runs as its own launch before, see wants_prenorm; TWO, the instantiation for M = 2, takes it itself,
+// and keeps every activation exact where F16 would not: gate|up at M = 2 20.5 us with that code and without);
 // the weights are the B operand, decoded exactly to F16. Each wave
 // keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5;
 // BF16 one, its tile is 16 chunks) and issues the next as soon
@@ -1206,6 +1207,14 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       for (int s = 0; s < SPC; ++s)
         xa[cc][s] = *reinterpret_cast<const uint4*>(stage + (m_row & 3) * ROWM_SLD + 2 * (cc * KC + xcol(s)));
   };
+  bool wide = false;                            // TWO: a token's slice spans more binades than one F16 operand holds
+  // a value of the lane's 8 columns further below the slice's exponent than that (p: stage_row's)
+  auto below = [&](const uint32_t (&vv)[4], int p) {
+    u16x2_t least = {0xFFFF, 0xFFFF};           // of the magnitudes less one: zeros come last
+#pragma unroll
+    for (int q = 0; q < 4; ++q) least = __builtin_elementwise_min(least, (u16x2_t)(__builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu) - (u16x2_t){1, 1}));
+    return (int)min((uint32_t)least.x, (uint32_t)least.y) + 1 < (p - (I4 ? 24 : 0) + 141 - 31) * 128;
+  };
   if constexpr (TWO) {
     // Two tokens: the fused norm here (one row load, one barrier among the waves), so the call stays one launch without
     // scratch. A wave's slice is one slice of the statistic, its order and the values those of norm_apply, bit for bit.
@@ -1224,14 +1233,48 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         norm_vec(v[t], 1.0f / sqrtf(ssq / (float)a.k + a.eps), w0, w1, v[t]);
       }
     }
+    if constexpr (BA) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if constexpr (BA) *reinterpret_cast<uint4*>(stage + t * ROWM_SLD + 16 * lane) = uint4{v[t][0], v[t][1], v[t][2], v[t][3]};
-      else ps[t] = stage_row(t, v[t]);          // in every lane; the k-group 0 lanes hold the two tokens' outputs
+      for (int t = 0; t < 2; ++t) *reinterpret_cast<uint4*>(stage + t * ROWM_SLD + 16 * lane) = uint4{v[t][0], v[t][1], v[t][2], v[t][3]};
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {             // 2^p in every lane; the k-group 0 lanes hold the two tokens' outputs
+        ps[t] = stage_row(t, v[t]);
+        wide |= __ballot(below(v[t], ps[t])) != 0;
+      }
     }
     wave_lds_sync();
     if (m_row < 2) take_rows();
     wave_lds_sync();
+    if constexpr (!BA) {
+      if (wide) {
+        // A slice that spans more than the 32 binades F16 holds (8-bit values down to 2^-17) takes the operand rows that
+        // two tokens leave idle: row 2L + t the values of token t whose exponent lies 32 L to 32 L + 31 below the
+        // slice's, by 2^(32 L - p): every value exact, as gemv_row has them. The rows' sums meet in tile_mma
+        const int p[2] = {ps[0] - (I4 ? 24 : 0), ps[1] - (I4 ? 24 : 0)};
+#pragma unroll 1
+        for (int grp = 0; grp < 4; ++grp) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = r & 1, lev = 2 * grp + (r >> 1);
+            f16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const int src = I4 ? int4_perm8(e) : e;
+              const uint32_t bits = (src & 1) ? v[t][src >> 1] >> 16 : v[t][src >> 1] & 0xFFFFu;
+              const int d = p[t] + 141 - max((int)(bits & 0x7FFFu) >> 7, 1);   // binades below the slice's exponent
+              o[e] = (max(d, 0) >> 5) == lev ? (f16_t)__builtin_amdgcn_ldexpf(bf16_bits_to_f32(bits), 32 * lev - p[t]) : (f16_t)0.0f;
+            }
+            *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
+          }
+          wave_lds_sync();
+          if ((m_row >> 2) == grp) take_rows();
+          wave_lds_sync();
+        }
+#pragma unroll
+        for (int i = 3; i >= 0; --i) ps[i] = ps[i & 1] - 32 * (2 * g + (i >> 1));
+      }
+    }
   } else {
 #pragma unroll 1
     for (int grp = 0; !BA && grp < ng; ++grp) {
@@ -1322,10 +1365,21 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       }
       __builtin_amdgcn_sched_barrier(0);      // decode chunk by chunk: keeps the decoded operands' registers few
     }
+    // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
     float* rp = red + wave * a.row_ld + jt * 256;
+    float o[4];
 #pragma unroll
-    for (int i = 0; i < (TWO ? 2 : 4); ++i)     // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
-      if (!TWO || g == 0) rp[(4 * g + i) * 16 + m_row] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
+    for (int i = 0; i < 4; ++i) o[i] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
+    if constexpr (TWO) {
+      if (wide) {                               // the two tokens' levels
+        o[0] = quad16_sum(o[0] + o[2]);
+        o[1] = quad16_sum(o[1] + o[3]);
+      }
+      if (g == 0) { rp[m_row] = o[0]; rp[16 + m_row] = o[1]; }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rp[(4 * g + i) * 16 + m_row] = o[i];
+    }
   };
   if constexpr (DEPTH == 1) {
     for (int j = 0; j < ntl; ++j) {

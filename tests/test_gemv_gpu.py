@@ -339,6 +339,13 @@ def test_gemv_rowm_small_beside_large(torch_gpu, fmt, mtok, rng):
     _small_beside_large(torch_gpu, fmt, mtok, (-30,), rng)
 
 
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
+def test_gemv_two_tokens_any_range(torch_gpu, fmt, rng):
+    """Two tokens keep every activation exact, however far below its slice's maximum (their operand rows are there for
+    it): 32 binades are one operand, 200 seven of them."""
+    _small_beside_large(torch_gpu, fmt, 2, (-31, -32, -60, -100, -200), rng)
+
+
 def _small_beside_large(torch, fmt, mtok, exps, rng):
     from monolith_mi355 import kernels
     k, big = 3072, 1000
@@ -354,7 +361,7 @@ def _small_beside_large(torch, fmt, mtok, exps, rng):
     w = _upload(torch, m)
     for exp in exps:
         x = rbf((1 + rng.random((mtok, k))) * np.where(rng.random((mtok, k)) < 0.5, -1, 1))
-        up = min(0, -110 - exp)                               # the small ones stay above 2^-110
+        up = min(0, exp + 110)                                # the small ones stay above 2^-110
         x = rbf(x * np.float32(2.0 ** (exp - up)))
         x[:, big] = rbf(np.float32(1.5 * 2.0 ** -up))
         xd = to_dev_bf16(torch, x)
@@ -363,6 +370,12 @@ def _small_beside_large(torch, fmt, mtok, exps, rng):
         ref = np.tile(x.astype(np.float64) @ wd.T, (1, rep))
         bound = np.tile(np.abs(x.astype(np.float64)) @ np.abs(wd).T, (1, rep))
         assert (np.abs(got - ref) <= 2.0 ** -18 * bound).all(), (fmt, mtok, exp)
+        if mtok == 2:                                         # the second token alone, the first of ordinary values
+            x[0] = rbf(rng.standard_normal(k).astype(np.float32))
+            got = kernels.gemv(w, to_dev_bf16(torch, x), out_f32=True).cpu().numpy().astype(np.float64)
+            ref = np.tile(x.astype(np.float64) @ wd.T, (1, rep))
+            bound = np.tile(np.abs(x.astype(np.float64)) @ np.abs(wd).T, (1, rep))
+            assert (np.abs(got - ref) <= 2.0 ** -18 * bound).all(), (fmt, exp)
 
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
