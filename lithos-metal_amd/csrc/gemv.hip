@@ -2336,10 +2336,11 @@ Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
   // a CU 56.5 / 64.1 / 78.4 us, of three 47.4 / 52.4 / 61.2 (gemv_tk 56.0 / 58.6 / 66.0, with partials); longer ones
   // 151936 x 2560 two rounds of one 44.6 / 50.4 / 62.4, of two 48.8 / 56.3 / 71.7 (gemv_tk 53.9 / 55.7 / 59.2). FP8 has no
   // other kernel. INT4 and BF16 stay on gemv_tk there: INT4 248320 x 2048 at M = 8 64.7 us against 88.6 here, 128256 x
-  // 3072 53.1 against 57.2, BF16 248320 x 5120 379 against 394.
+  // 3072 53.1 against 57.2, BF16 248320 x 5120 379 against 394. So does NVFP4 where K is split too: gemv_tk needs less
+  // scratch for it.
   const long long most = (long long)(kMaxLds - fixed) / (S * 1024LL);
   if (n_tiles > G * most) {
-    if (d->format == FMT_INT4 || d->format == FMT_BF16) return best;
+    if (d->format == FMT_INT4 || d->format == FMT_BF16 || (ks > 1 && d->format != FMT_FP8)) return best;
     const int res = S <= 4 ? std::max(per_cu, 1) : 1;
     const long long slot = std::max<long long>(1, (long long)cu_count() * res / ks), hold = slot * (most / res);
     G = (int)std::min<long long>(n_tiles, slot * ((n_tiles + hold - 1) / hold));
@@ -2354,6 +2355,7 @@ Plan plan_rowm(const mi_gemv_desc* d, int chunks, int n_tiles) {
 }
 
 Plan make_plan_fused(const mi_gemv_desc* d);
+size_t split_bytes(const mi_gemv_desc* d, const Plan& p);
 
 // split-K workspace: a fixed region of per-tile arrival counters (the same for every shape, so partials of one call
 // never land on the counters of another), then the FP32 partials [ks][m][n_tiles·16], then (prenorm) the
@@ -2474,6 +2476,15 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
   }
   if (rows > 2 && !pin_tk) {
     const Plan p = plan_rowm(d, chunks, n_tiles);
+    // a K that gemv_rowm splits (over 6144): BF16, INT4 and an NVFP4 K of no whole slices stay on gemv_tk where that needs
+    // less scratch: a caller's workspace or a stream captured before its first eager call may have no more, and what
+    // writes none can overlap. (BF16 at M = 3 and 4 over tens of thousands of rows, which gemv_tk does not split: 34816 x
+    // 8192 123 us there, 90 here with two splits; a program that gives such a call room has MI_GEMV_KERNEL=rowm)
+    const bool lean = p.kernel && p.ks > 1 && !pin_rowm && (fmt == FMT_BF16 || fmt == FMT_INT4 || (fmt == FMT_NVFP4 && chunks % 4));
+    if (lean) {
+      const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
+      if (t.kernel && split_bytes(d, t) < split_bytes(d, p)) return t;
+    }
     if (p.kernel) return p;
   }
   return plan_tk(d, fmt, chunks, n_tiles, groups, rows);
