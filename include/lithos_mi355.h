@@ -456,8 +456,10 @@ typedef struct mi_sample_desc {
   uint64_t seed;
   uint32_t step;
   const mi_step_state* state; /* optional: seed and step from the step state */
-  void* workspace;            /* optional, mi_sample_workspace_bytes, zeroed once before its first use (the
-                                 arrival counters are left at zero by every call); NULL: the library's own */
+  void* workspace;            /* optional, at least mi_sample_workspace_bytes, zeroed once before its first use (the
+                                 arrival counters are left at zero by every call). From 1 KiB + t·(8·ceil(vocab / 2048) +
+                                 131200·max(4, ceil(vocab / 65528))) bytes on, several workgroups count a row, as with
+                                 NULL: the library's own */
   size_t workspace_bytes;
 } mi_sample_desc;
 size_t mi_sample_workspace_bytes(const mi_sample_desc* d);

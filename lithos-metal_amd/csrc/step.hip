@@ -39,8 +39,11 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
 
 // The order "larger value, then lower index" over the numbers is total, so combining partial results in any order
 // gives the same answer: the spans of a row run in parallel and the last one to finish folds them.
-constexpr int ARGMAX_SPAN = ARGMAX_THREADS * 8;    // logits per workgroup
-constexpr int ARGMAX_MAX_SPANS = 512;
+// Logits per workgroup: 16 a thread. (8 a thread, twice the workgroups, publishing twice the partials: rows of 248320 x 1 /
+// 4 / 16 5.7 / 9.7 / 26.8 us, 16 a thread 5.4 / 7.4 / 16.1. Only a draw for one or two rows is faster with 8, its noise is
+// work for every logit: 248320 28.0 → 27.2 us, see sample_layout)
+constexpr int ARGMAX_SPAN = ARGMAX_THREADS * 16;
+constexpr int ARGMAX_MAX_SPANS = 256;
 constexpr size_t ARGMAX_COUNTERS = 256;            // bytes: 16 per-row arrival counters, padded
 
 __device__ __forceinline__ void st_dev8(unsigned long long* p, unsigned long long v) {
@@ -111,8 +114,9 @@ __device__ __forceinline__ T wave_total(T v) {
 }
 
 // A row's counts as sample_threshold's last workgroup holds them: 16 bits a key in LDS, and the few carries past them
-// (at most vocab / 65536: keys that hold more than 65535 logits)
-constexpr int MAX_CARRY = 16;
+// (each at least 32768 logits of a row of at most 2^20)
+constexpr int MAX_CARRY = 32;
+constexpr int CARRY_SPAN = 32760;                          // logits one workgroup counts between two sweeps of carries
 struct KeyCounts {
   const uint16_t* h;
   const uint32_t* carry_key;
@@ -120,7 +124,7 @@ struct KeyCounts {
   int n_carry;
   __device__ __forceinline__ uint32_t operator()(uint32_t k) const {
     uint32_t c = h[k];
-    for (int i = 0; i < n_carry; ++i) c += carry_key[i] == k ? carry[i] << 16 : 0u;
+    for (int i = 0; i < n_carry; ++i) c += carry_key[i] == k ? carry[i] : 0u;
     return c;
   }
 };
@@ -233,32 +237,54 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_threshold(const uint16_
     const uint32_t k = key16(bits);
     atomicAdd(&h16[k >> 1], (k & 1u) ? 0x10000u : 1u);
   };
-  const int nv = (reinterpret_cast<uintptr_t>(p) & 15) == 0 ? n / 8 : 0;   // whole 16-byte vectors of an aligned row
-  constexpr int UN = 4;                                                    // vectors in flight per thread
-  for (int v0 = tid; v0 < nv; v0 += UN * SELECT_THREADS) {
-    uint4 q[UN];
+  auto count_span = [&](const uint16_t* p, int n) {
+    const int nv = (reinterpret_cast<uintptr_t>(p) & 15) == 0 ? n / 8 : 0;   // whole 16-byte vectors of an aligned row
+    constexpr int UN = 4;                                                    // vectors in flight per thread
+    for (int v0 = tid; v0 < nv; v0 += UN * SELECT_THREADS) {
+      uint4 q[UN];
 #pragma unroll
-    for (int i = 0; i < UN; ++i) q[i] = reinterpret_cast<const uint4*>(p)[min(v0 + i * SELECT_THREADS, nv - 1)];
+      for (int i = 0; i < UN; ++i) q[i] = reinterpret_cast<const uint4*>(p)[min(v0 + i * SELECT_THREADS, nv - 1)];
 #pragma unroll
-    for (int i = 0; i < UN; ++i) {
-      if (v0 + i * SELECT_THREADS >= nv) break;
-      const uint32_t qw[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
+      for (int i = 0; i < UN; ++i) {
+        if (v0 + i * SELECT_THREADS >= nv) break;
+        const uint32_t qw[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        count(qw[e] & 0xFFFFu);
-        count(qw[e] >> 16);
+        for (int e = 0; e < 4; ++e) {
+          count(qw[e] & 0xFFFFu);
+          count(qw[e] >> 16);
+        }
       }
     }
-  }
-  for (int c = 8 * nv + tid; c < n; c += 8 * SELECT_THREADS) {             // the rest, or an unaligned row
-    uint16_t b[8];
+    for (int c = 8 * nv + tid; c < n; c += 8 * SELECT_THREADS) {             // the rest, or an unaligned row
+      uint16_t b[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) b[i] = p[min(c + i * SELECT_THREADS, n - 1)];
+      for (int i = 0; i < 8; ++i) b[i] = p[min(c + i * SELECT_THREADS, n - 1)];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (c + i * SELECT_THREADS < n) count(b[i]);
+      for (int i = 0; i < 8; ++i)
+        if (c + i * SELECT_THREADS < n) count(b[i]);
+    }
+    __syncthreads();
+  };
+  // a row in one workgroup (no room for more in the workspace): the counts from 32768 on go to the carries between spans
+  const int sub = n > SELECT_SPAN_MAX ? CARRY_SPAN : n;
+#pragma unroll 1
+  for (int at = 0;;) {
+    count_span(p + at, min(sub, n - at));
+    at += sub;
+    if (at >= n) break;
+    for (int i = 0; i < KEY_BLOCK / 2; ++i) {
+      const int word = tid * (KEY_BLOCK / 2) + ((i + tid) & (KEY_BLOCK / 2 - 1));
+      const uint32_t c = h16[word];
+      if (!(c & 0x80008000u)) continue;
+      h16[word] = c & 0x7FFF7FFFu;
+      for (int e = 0; e < 2; ++e)
+        if ((c >> (16 * e + 15)) & 1u) {
+          const uint32_t slot = atomicAdd(&n_carry, 1u);
+          if (slot < MAX_CARRY) { carry_key[slot] = 2 * word + e; carry[slot] = 32768u; }
+        }
+    }
+    __syncthreads();
   }
-  __syncthreads();
 
   if (nb > 1) {
     // ---- publish: thread b the block of keys 64·b .. + 63, its 16 words in an order rotated by the thread (no bank
@@ -342,7 +368,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_threshold(const uint16_
             for (int e = 0; e < 4; ++e)
               if (c[e] >> 16) {
                 const uint32_t slot = atomicAdd(&n_carry, 1u);
-                if (slot < MAX_CARRY) { carry_key[slot] = 4 * word + e; carry[slot] = c[e] >> 16; }
+                if (slot < MAX_CARRY) { carry_key[slot] = 4 * word + e; carry[slot] = c[e] & 0xFFFF0000u; }
               }
           }
         }
@@ -431,17 +457,17 @@ __global__ __launch_bounds__(SELECT_THREADS) void sample_threshold(const uint16_
   if (tid == 0) tau[row] = fmaxf(fmaxf(tau_k, tau_p), tau_m);
 }
 
-// grid (spans, rows): each workgroup scans ARGMAX_SPAN logits of one row with 16-byte loads, publishes its best,
+// grid (spans, rows): each workgroup scans `span` logits of one row with 16-byte loads, publishes its best,
 // and the last workgroup of the row to arrive folds the row's partials and resets the row's counter. SAMPLE: the
 // value of a BF16 logit v >= tau is v / temperature + its Gumbel noise, any other logit is left out.
 template <bool SAMPLE>
-__global__ __launch_bounds__(ARGMAX_THREADS) void argmax_spans(mi_argmax_desc d, uint32_t* counters,
+__global__ __launch_bounds__(ARGMAX_THREADS) void argmax_spans(mi_argmax_desc d, int span, uint32_t* counters,
                                                                unsigned long long* part, SampleCtx sc) {
   __shared__ float sv[ARGMAX_THREADS / 64];
   __shared__ int si[ARGMAX_THREADS / 64];
   __shared__ int last;
   const int row = blockIdx.y, nb = gridDim.x, tid = threadIdx.x;
-  const int lo = blockIdx.x * ARGMAX_SPAN, hi = min(lo + ARGMAX_SPAN, d.vocab);
+  const int lo = blockIdx.x * span, hi = min(lo + span, d.vocab);
   float bv = -INFINITY;
   int bi = 0x7FFFFFFF;
   float th = 0.0f;
@@ -561,6 +587,9 @@ __global__ __launch_bounds__(64) void advance_step(mi_advance_desc d) {
 }
 
 int argmax_spans_of(int vocab) { return (vocab + ARGMAX_SPAN - 1) / ARGMAX_SPAN; }
+
+// the 8-byte partials of a workspace that starts on 4 bytes lie 4 before where they would (the counters end long before)
+char* down8(void* ws) { return reinterpret_cast<char*>(reinterpret_cast<uintptr_t>(ws) & ~(uintptr_t)7); }
 
 // sample_threshold's workgroups per row and the logits each counts (a multiple of 8: rows stay 16-byte aligned)
 int select_span_of(int vocab, int* wgs) {
@@ -808,29 +837,47 @@ int mi_argmax(const mi_argmax_desc* d, void* stream) {
     return rc;
   }
   auto* counters = static_cast<uint32_t*>(ws);
-  auto* part = reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + ARGMAX_COUNTERS);
+  auto* part = reinterpret_cast<unsigned long long*>(down8(ws) + ARGMAX_COUNTERS);
   hipLaunchKernelGGL(argmax_spans<false>, dim3(nb, d->t), dim3(ARGMAX_THREADS), 0, static_cast<hipStream_t>(stream),
-                     *d, counters, part, SampleCtx{});
+                     *d, ARGMAX_SPAN, counters, part, SampleCtx{});
   MI_TRY_HIP(hipGetLastError(), "argmax launch");
   return MI_OK;
 }
 
 // workspace: argmax counters (16, then sample_threshold's 16) | partials | tau[16] | per (row, workgroup of
 // sample_threshold): the maps of its key blocks [16] u64 | the blocks' 16-bit counts [1024][64]
-size_t sample_layout(int t, int vocab, size_t* off_tau, size_t* off_map, size_t* off_part) {
-  const size_t part = ARGMAX_COUNTERS + (size_t)t * argmax_spans_of(vocab) * sizeof(unsigned long long);
-  int wgs = 0;
-  (void)select_span_of(vocab, &wgs);
-  *off_tau = (part + 255) / 256 * 256;
-  *off_map = *off_tau + 256;
-  *off_part = *off_map + (size_t)t * wgs * SELECT_WAVES * sizeof(unsigned long long);
-  return *off_part + (size_t)t * wgs * SELECT_THREADS * PART_U64 * sizeof(unsigned long long);
+struct SampleLayout {
+  int span, wgs;                // the draw's logits per workgroup, sample_threshold's workgroups per row and their span
+  int count_span;
+  size_t off_tau, off_map, off_part, bytes;
+};
+SampleLayout sample_layout(int t, int vocab) {
+  SampleLayout l{};
+  l.span = t <= 2 ? ARGMAX_SPAN / 2 : ARGMAX_SPAN;
+  l.count_span = select_span_of(vocab, &l.wgs);
+  l.off_tau = (ARGMAX_COUNTERS + (size_t)t * ((vocab + l.span - 1) / l.span) * sizeof(unsigned long long) + 255) / 256 * 256;
+  l.off_map = l.off_tau + 256;
+  l.off_part = l.off_map + (size_t)t * l.wgs * SELECT_WAVES * sizeof(unsigned long long);
+  l.bytes = l.off_part + (size_t)t * l.wgs * SELECT_THREADS * PART_U64 * sizeof(unsigned long long);
+  return l;
+}
+// The least that a call takes, what it asks callers for: 256 KB a row, where the workgroups' counts need 128 KB each and
+// at least four. With less than sample_layout's bytes one workgroup counts a row (nothing to publish): 248320 logits
+// 27 → 50 us with the draw, 32000 as fast
+SampleLayout sample_least(int t, int vocab) {
+  SampleLayout l{};
+  l.span = ARGMAX_SPAN;
+  l.wgs = 1;
+  l.count_span = vocab;
+  l.off_tau = (ARGMAX_COUNTERS + (size_t)t * argmax_spans_of(vocab) * sizeof(unsigned long long) + 255) / 256 * 256;
+  l.off_map = l.off_part = l.off_tau + 256;
+  l.bytes = l.off_part + (size_t)t * HIST_KEYS * sizeof(uint32_t);
+  return l;
 }
 
 size_t mi_sample_workspace_bytes(const mi_sample_desc* d) {
   if (!d || d->t < 1 || d->vocab < 1) return 0;
-  size_t a, b, c;
-  return sample_layout(d->t, d->vocab, &a, &b, &c);
+  return sample_least(d->t, d->vocab).bytes;
 }
 
 int mi_sample(const mi_sample_desc* d, void* stream) {
@@ -838,20 +885,22 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
   MI_REQUIRE(d->t >= 1 && d->t <= 16 && d->vocab > 0 && d->ld >= d->vocab, "mi_sample: bad shape");
   MI_REQUIRE(d->temperature > 0.0f && d->top_k >= 0 && d->top_p >= 0.0f && d->min_p >= 0.0f,
              "mi_sample: temperature > 0, top_k / top_p / min_p >= 0 (temperature 0 is mi_argmax)");
-  const int nb = argmax_spans_of(d->vocab);
-  MI_REQUIRE(nb <= ARGMAX_MAX_SPANS, "mi_sample: vocab %d exceeds %d", d->vocab, ARGMAX_MAX_SPANS * ARGMAX_SPAN);
-  size_t off_tau, off_map, off_part;
-  const size_t need = sample_layout(d->t, d->vocab, &off_tau, &off_map, &off_part);
+  MI_REQUIRE(argmax_spans_of(d->vocab) <= ARGMAX_MAX_SPANS, "mi_sample: vocab %d exceeds %d", d->vocab,
+             ARGMAX_MAX_SPANS * ARGMAX_SPAN);
+  SampleLayout l = sample_layout(d->t, d->vocab);
+  const SampleLayout least = sample_least(d->t, d->vocab);
   void* ws = d->workspace;
   if (ws) {
-    MI_REQUIRE(d->workspace_bytes >= need, "mi_sample: workspace %zu B < %zu B", d->workspace_bytes, need);
-  } else if (int rc = mi_library_scratch(MI_SCRATCH_ARGMAX, need, static_cast<hipStream_t>(stream), &ws)) {
-    return rc;
+    MI_REQUIRE(d->workspace_bytes >= least.bytes, "mi_sample: workspace %zu B < %zu B", d->workspace_bytes, least.bytes);
+    if (d->workspace_bytes < l.bytes) l = least;
+  } else if (mi_library_scratch(MI_SCRATCH_ARGMAX, l.bytes, static_cast<hipStream_t>(stream), &ws)) {
+    l = least;                                      // it cannot grow (a capture): what it holds may be enough
+    if (int rc = mi_library_scratch(MI_SCRATCH_ARGMAX, l.bytes, static_cast<hipStream_t>(stream), &ws)) return rc;
   }
-  char* wb = static_cast<char*>(ws);
-  auto* counters = reinterpret_cast<uint32_t*>(wb);
+  char* wb = down8(ws);
+  auto* counters = static_cast<uint32_t*>(ws);
   auto* part = reinterpret_cast<unsigned long long*>(wb + ARGMAX_COUNTERS);
-  auto* tau = reinterpret_cast<float*>(wb + off_tau);
+  auto* tau = reinterpret_cast<float*>(wb + l.off_tau);
   uint32_t flags = 0;
   if (d->top_k > 0) flags |= 1u;
   if (d->top_p > 0.0f && d->top_p < 1.0f) flags |= 2u;
@@ -859,8 +908,6 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
   if (d->topp_in_topk) flags |= 8u;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (flags & 7u) {
-    int wgs = 0;
-    const int span = select_span_of(d->vocab, &wgs);
     const size_t lds = HIST_KEYS / 2 * sizeof(uint32_t);
     static std::once_flag once;                     // more than 64 KB of dynamic LDS must be allowed once
     std::call_once(once, [&] {
@@ -868,9 +915,9 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       (void)hipGetLastError();
     });
-    hipLaunchKernelGGL(sample_threshold, dim3(wgs, d->t), dim3(SELECT_THREADS), lds, s, d->logits, d->ld, d->vocab, span,
-                       counters + 16, reinterpret_cast<unsigned long long*>(wb + off_map),
-                       reinterpret_cast<unsigned long long*>(wb + off_part), tau, d->top_k, d->temperature, d->top_p,
+    hipLaunchKernelGGL(sample_threshold, dim3(l.wgs, d->t), dim3(SELECT_THREADS), lds, s, d->logits, d->ld, d->vocab, l.count_span,
+                       counters + 16, reinterpret_cast<unsigned long long*>(wb + l.off_map),
+                       reinterpret_cast<unsigned long long*>(wb + l.off_part), tau, d->top_k, d->temperature, d->top_p,
                        d->min_p, flags);
   } else {
     tau = nullptr;                                  // nothing to cut: keep every logit
@@ -878,7 +925,8 @@ int mi_sample(const mi_sample_desc* d, void* stream) {
   mi_argmax_desc am{};
   am.t = d->t; am.vocab = d->vocab; am.logits = d->logits; am.ld = d->ld; am.f32 = 0; am.ids = d->ids;
   SampleCtx sc{tau, 1.0f / d->temperature, (uint32_t)d->seed, (uint32_t)(d->seed >> 32), d->step, d->state};
-  hipLaunchKernelGGL(argmax_spans<true>, dim3(nb, d->t), dim3(ARGMAX_THREADS), 0, s, am, counters, part, sc);
+  hipLaunchKernelGGL(argmax_spans<true>, dim3((d->vocab + l.span - 1) / l.span, d->t), dim3(ARGMAX_THREADS), 0, s, am, l.span, counters,
+                     part, sc);
   MI_TRY_HIP(hipGetLastError(), "sample launch");
   return MI_OK;
 }

@@ -580,3 +580,63 @@ def test_sample_threshold_spans(torch_gpu, vocab, opts):
     for step in (0, 3):
         tok = kernels.sample(lb, seed=77, step=step, temperature=0.8, **opts).cpu().tolist()
         assert tok == [O.sample(lf[i], seed=77, step=step, t=i, temperature=0.8, **opts) for i in range(3)]
+
+
+@pytest.mark.parametrize("vocab", [9, 65537, 248320, 300001, 1 << 20])
+@pytest.mark.parametrize("opts", [dict(top_k=5), dict(top_p=0.7), dict(top_k=70000, top_p=0.9, topp_in_topk=True)],
+                         ids=["k", "p", "kp"])
+def test_sample_in_a_caller_workspace(torch_gpu, vocab, opts):
+    """The least workspace (256 KB a row, the partials of spans of 4096 logits and 1 KiB at most: one workgroup counts a
+    row, its counts past 32767 in carries), one that holds the counts of several, and either at 4 bytes past an 8-byte
+    boundary: the oracle's draws, call after call; one byte less than the least is refused."""
+    import ctypes as C
+    torch = torch_gpu
+    from monolith_mi355.runtime import hip
+    _say("sample workspace", vocab, opts)
+    rng = np.random.default_rng(vocab + 1)
+    rows = np.zeros((3, vocab), np.float32)
+    rows[0] = rng.standard_normal(vocab) * 3.0
+    rows[1] = -1.25
+    rows[2] = rng.integers(0, 3, vocab)                           # three keys
+    lb = to_dev_bf16(torch, rows)
+    lf = from_dev_bf16(lb)
+    t = 3
+    ids = torch.empty(t, dtype=torch.int32, device="cuda")
+    d = hip.MiSampleDesc(t=t, vocab=vocab, logits=hip.ptr(lb), ld=lb.stride(0), ids=hip.ptr(ids), temperature=0.8, seed=77,
+                         **{k: int(v) if k == "topp_in_topk" else v for k, v in opts.items()})
+    least = hip.load().mi_sample_workspace_bytes(C.byref(d))
+    assert least == -(-(256 + t * -(-vocab // 4096) * 8) // 256) * 256 + 256 + t * 262144
+    full = 1024 + t * (8 * -(-vocab // 2048) + 131200 * max(4, -(-vocab // 65528)))
+    ref = {step: [O.sample(lf[i], seed=77, step=step, t=i, temperature=0.8, **opts) for i in range(t)] for step in (0, 3)}
+    for nbytes in (least, max(least, full)):
+        for off in (0, 4):
+            ws = torch.zeros(nbytes + off, dtype=torch.uint8, device="cuda")[off:]
+            d.workspace, d.workspace_bytes = hip.ptr(ws), nbytes
+            for step in (0, 3, 0):
+                d.step = step
+                hip.call("mi_sample", C.byref(d), hip.stream_handle(None))
+                assert ids.cpu().tolist() == ref[step], (nbytes == least, off, step)
+            assert not ws[:128].any()                             # counters back at zero
+    d.workspace_bytes = least - 1
+    with pytest.raises(hip.MiError):
+        hip.call("mi_sample", C.byref(d), hip.stream_handle(None))
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_argmax_workspace_at_four_bytes(torch_gpu, f32):
+    """The partials of spans of 4096 logits and 256 bytes are enough, also 4 bytes past an 8-byte boundary."""
+    import ctypes as C
+    torch = torch_gpu
+    from monolith_mi355.runtime import hip
+    t, vocab = 5, 70000
+    x = torch.randn(t, vocab, device="cuda").to(torch.float32 if f32 else torch.bfloat16)
+    ids = torch.empty(t, dtype=torch.int32, device="cuda")
+    need = 256 + t * -(-vocab // 4096) * 8
+    ws = torch.zeros(need + 4, dtype=torch.uint8, device="cuda")[4:]
+    d = hip.MiArgmaxDesc(t=t, vocab=vocab, logits=hip.ptr(x), ld=vocab, f32=int(f32), ids=hip.ptr(ids),
+                         workspace=hip.ptr(ws), workspace_bytes=need)
+    assert hip.load().mi_argmax_workspace_bytes(C.byref(d)) == need
+    for _ in range(2):
+        x.normal_()
+        hip.call("mi_argmax", C.byref(d), hip.stream_handle(None))
+        assert ids.cpu().tolist() == O.argmax(x.float().cpu().numpy()).tolist()
