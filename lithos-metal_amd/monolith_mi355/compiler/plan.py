@@ -303,6 +303,14 @@ def fuse_gdn(p: Plan, defer_max_t: int = 2) -> None:
         p.bump("fuse_gdn")
 
 
+def _matrix_of(p: Plan, op: POp) -> Tuple[str, int, int]:
+    """(format, rows, K) of the matrix a GEMV launch streams: its slab's, the rows of all slabs where it was merged."""
+    w = op.inputs[1]
+    s = p.slabs.get(w.name)
+    fmt, n, k = (s["format"], s["n"] * s.get("experts", 1), s["k"]) if s else (w.format or "nvfp4", *p.shape(w)[:2])
+    return fmt, int(op.attrs.get("n_rows", n)), int(k)
+
+
 def fold_gdn_conv(p: Plan) -> None:
     """At T <= 2 the GDN short conv moves into the input projection's epilogue (``mi_gemv_desc.conv_*``): the GEMV
     that produces the step's q|k|v rows convolves each of them where it is computed and writes the convolved values
@@ -321,7 +329,7 @@ def fold_gdn_conv(p: Plan) -> None:
         prod = next((o for o in p.ops if o.kind == "gemv" and o.outputs[0].name == root), None)
         if prod is None or prod.attrs.get("epilogue") is not None or prod.attrs.get("row_range") is not None:
             continue
-        if p.t == 2 and two_tokens_on_matrix_cores(prod.inputs[1].format or "nvfp4", *p.shape(prod.inputs[1])[:2]):
+        if p.t == 2 and two_tokens_on_matrix_cores(*_matrix_of(p, prod)):
             continue
         n_main = 1 + max(idx for idx, _, _ in ps.values())
         cs = op.inputs[n_main]

@@ -24,6 +24,9 @@ last NVFP4 group (K not a multiple of 1024 columns), padded to 8 or 16 bytes per
 
 from __future__ import annotations
 
+import ctypes as C
+import functools
+import os
 from dataclasses import dataclass
 from typing import Optional, Tuple
 
@@ -63,10 +66,20 @@ def pack_bytes(fmt: str, n: int, k: int) -> int:
 
 
 def two_tokens_on_matrix_cores(fmt: str, n: int, k: int) -> bool:
-    """Whether a dense GEMV of two tokens runs on the matrix-core kernel (many weights, a long K in one split; the same
-    rule and its figures: ``csrc/gemv.hip`` ``rowm_at_two``); the Gated DeltaNet conv then stays out of its epilogue."""
-    least = (40 if fmt == "fp8_e4m3" else 20) << 20
-    return pack_bytes(fmt, n, k) >= least and (2048 if fmt == "bf16" else 3072) <= k <= 6144
+    """Whether a dense GEMV of two tokens runs on the matrix-core kernel, as its planner says (``mi_gemv_plan``: many
+    weights, a long K in one split, unless the environment pins a kernel); the Gated DeltaNet conv then stays out of its
+    epilogue."""
+    return _two_tokens_plan(fmt, n, k, tuple(map(os.environ.get, ("MI_GEMV_KERNEL", "MI_GEMV_ROW", "MI_GEMV_ROWM",
+                                                                  "MI_GEMV_ROWM_K")))) == 3
+
+
+@functools.lru_cache(maxsize=256)
+def _two_tokens_plan(fmt: str, n: int, k: int, pins) -> int:
+    from ..runtime import hip
+    out = (C.c_int32 * 7)()
+    d = hip.MiGemvDesc(format=hip.MI_FMT[fmt], n=n, k=k, m=2, w=256, x=256, ldx=k, y=256, ldy=n)   # nothing is read
+    hip.call("mi_gemv_plan", C.byref(d), out)
+    return out[0]
 
 
 @dataclass

@@ -210,6 +210,34 @@ def test_emit_without_adjacency_keeps_the_reference_split(tmp_path):
     assert comb.meta["desc"]["top_k"] == 8 and comb.meta["desc"]["ld_gate"] > 0
 
 
+@pytest.mark.parametrize("z_rows,qkv_rows,k,folds", [(6144, 10240, 5120, False),   # 47 MB in all, 17.7 the first slab
+                                                       (6144, 640, 5120, True),       # 19.5 MB in all
+                                                       (6144, 10240, 2048, True)])    # a short K
+def test_conv_fold_at_two_tokens_counts_every_merged_slab(z_rows, qkv_rows, k, folds):
+    """At T = 2 the conv folds into the input projection unless its launch, over the rows of all merged slabs, runs on
+    the matrix cores."""
+    from monolith_mi355.compiler.plan import Plan, POp, PVal, fold_gdn_conv, merge_adjacent_slabs
+    from monolith_mi355.formats.pack import pack_bytes
+    slabs, off = {}, 0
+    for name, n in (("z", z_rows), ("qkv", qkv_rows)):
+        nb = pack_bytes("nvfp4", n, k)
+        slabs[name] = dict(format="nvfp4", n=n, k=k, experts=1, offset=off, nbytes=nb)
+        off += nb
+    h = PVal("h", (2, k), "bf16")
+    w = {n: PVal(n, (s["n"], k), "u8", is_weight=True) for n, s in slabs.items()}
+    y = {n: PVal(n + ".y", (2, s["n"]), "bf16") for n, s in slabs.items()}
+    cs, taps, o = PVal("conv_state", (2, qkv_rows, 3), "bf16"), PVal("taps", (qkv_rows, 4), "bf16"), PVal("o", (2, 128), "bf16")
+    hv = (qkv_rows - 512) // 128
+    ops = [POp("gemv", [h, w["z"]], [y["z"]], {}), POp("gemv", [h, w["qkv"]], [y["qkv"]], {}),
+           POp("gdn_mixer", [h, y["qkv"], cs, cs, taps], [o],
+               dict(proj_segments={"in_proj_qkv": (1, 0, qkv_rows)}, k_heads=2, v_heads=hv, dk=128, dv=128))]
+    p = Plan(ops, 2, {v.name: v for v in (h, cs, taps, o, *w.values(), *y.values())}, {}, slabs)
+    merge_adjacent_slabs(p)
+    assert len(p.ops) == 2 and p.ops[0].attrs["n_rows"] == z_rows + qkv_rows
+    fold_gdn_conv(p)
+    assert ("conv" in p.ops[0].attrs) == folds == bool(p.report.get("fold_gdn_conv"))
+
+
 def test_emit_speculative_round(tmp_path):
     """The speculative program (T = 1 + γ): the verify pass writes the GDN state's second slot, then the accept scan,
     the commit pass (in place, the accepted count from the step state), the draft lookup and the verify select."""
