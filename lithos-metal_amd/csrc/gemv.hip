@@ -2479,8 +2479,8 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
     // a K that gemv_rowm splits (over 6144): BF16, INT4 and an NVFP4 K of no whole slices stay on gemv_tk where that needs
     // less scratch: a caller's workspace or a stream captured before its first eager call may have no more, and what
     // writes none can overlap. (BF16 at M = 3 and 4 over tens of thousands of rows, which gemv_tk does not split: 34816 x
-    // 8192 123 us there, 90 here with two splits; a program that gives such a call room has MI_GEMV_KERNEL=rowm)
-    const bool lean = p.kernel && p.ks > 1 && !pin_rowm && (fmt == FMT_BF16 || fmt == FMT_INT4 || (fmt == FMT_NVFP4 && chunks % 4));
+    // 8192 123 us there, 90 here with two splits)
+    const bool lean = p.kernel && p.ks > 1 && !pin_rowm && !getenv("MI_GEMV_ROWM") && (fmt == FMT_BF16 || fmt == FMT_INT4 || (fmt == FMT_NVFP4 && chunks % 4));
     if (lean) {
       const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
       if (t.kernel && split_bytes(d, t) < split_bytes(d, p)) return t;

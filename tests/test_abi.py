@@ -60,7 +60,7 @@ def test_gemv_plans_fit_the_hardware(n, k, m):
     hip.call("mi_gemv_plan", C.byref(_desc(hip, n=n, k=k, m=m, ldx=k, ldy=n)), out)
     kernel, waves, kw, tb, ks, lds, wgs = list(out)
     chunks = k // 128
-    # gemv_row (VALU) for M <= 2; gemv_rowm (MFMA, 4-chunk K slices) above when its slices fit, else gemv_tk
+    # gemv_row (VALU) for M <= 2; gemv_rowm (MFMA) above from one slice of K (4 chunks) on, else gemv_tk
     assert kernel == (1 if m <= 2 else 3 if chunks % 4 == 0 else 2)
     assert 1 <= waves <= 16 and kw >= 1 and lds <= 160 * 1024 and wgs >= 1 and ks >= 1 and tb >= 1
     if kernel == 1:                                      # K splits of ≤ waves·kw chunks each

@@ -254,26 +254,27 @@ def test_gemv_gated_head_norm(torch_gpu, fmt, mtok, plan, rng, monkeypatch):
     assert chk.ok_rounded() and chk.within, (fmt, mtok, plan, chk)
 
 
-@pytest.mark.parametrize("fmt", ["nvfp4", "fp8_e4m3", "int4_affine"])
+@pytest.mark.parametrize("fmt", ["nvfp4", "fp8_e4m3", "int4_affine", "bf16"])
 @pytest.mark.parametrize("mtok", [3, 8, 16])
 @pytest.mark.parametrize("n,k,plan", [(1040, 2048, None), (1040, 2048, "1,3"), (336, 6144, "2,1"),
                                       (336, 6144, "3,2"), (5120, 17408, None)])
 @pytest.mark.parametrize("epi", [None, "residual", "silu_mul"])
 def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch):
-    """The M >= 3 kernel (K slices per wave on the matrix cores, several tiles per workgroup; NVFP4, FP8, INT4) over
+    """The M >= 3 kernel (K slices per wave on the matrix cores, several tiles per workgroup) over
     forced K splits and tiles per workgroup, against the oracle."""
     from monolith_mi355 import kernels
     if plan:
         monkeypatch.setenv("MI_GEMV_ROWM", plan)
-    if fmt == "int4_affine":                       # INT4 takes gemv_rowm only when it is pinned
-        monkeypatch.setenv("MI_GEMV_KERNEL", "rowm")
     m = _matrix(fmt, n, k, rng)
     x = rbf(rng.standard_normal((mtok, k)))
     res = rbf(rng.standard_normal((mtok, n)))
     kw = dict(epilogue=epi)
     if epi == "residual":
         kw["residual"] = to_dev_bf16(torch_gpu, res)
-    got = from_dev_bf16(kernels.gemv(_upload(torch_gpu, m), to_dev_bf16(torch_gpu, x), **kw))
+    w, xd = _upload(torch_gpu, m), to_dev_bf16(torch_gpu, x)
+    launch = _plan(w, xd, **kw)
+    assert launch[0] == 3 and (not plan or plan[0] == "1" or launch[4] == int(plan[0])), launch
+    got = from_dev_bf16(kernels.gemv(w, xd, **kw))
     wd = _dequant(m)
     if epi == "silu_mul":
         ref = ON.linear(x, wd[np.argsort(ON.interleave_chunks(n // 2, n // 2, 8))], epilogue="silu_mul")
@@ -287,10 +288,12 @@ def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch
 @pytest.mark.parametrize("mtok", [3, 4, 5, 8, 9, 13, 16])
 @pytest.mark.parametrize("n,k", [(24, 128), (4117, 640), (56, 896), (33, 1792), (40, 6656)])
 def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
-    """Every remainder of the four rows staged at a time, a slice of one chunk, one more tile than workgroups, two K
-    splits; a row of zeros, one scaled by 2^60 and one by 2^-60 (each row's own power-of-two prescale): every row
-    inside the leaf gate of its own values."""
+    """Every remainder of the four rows staged at a time, a slice of one chunk, two K splits, one tile a workgroup (NVFP4
+    under a slice of K runs on gemv_tk, small BF16 in token passes on gemv_row); a row of zeros, one scaled by 2^60 and
+    one by 2^-60 (each row's own power-of-two prescale): every row inside the leaf gate of its own values."""
     m = _matrix(fmt, n, k, rng)
+    launch = _plan(_upload(torch_gpu, m), to_dev_bf16(torch_gpu, np.zeros((mtok, k), np.float32)))
+    assert launch[0] == (2 if fmt == "nvfp4" and k < 512 else 1 if fmt == "bf16" and n * k * 2 <= 256 << 10 else 3)
     x = rbf(rng.standard_normal((mtok, k)).astype(np.float32))
     x[0] = 0.0
     x[1] *= 2.0 ** 60
@@ -302,6 +305,28 @@ def test_gemv_rowm_edges(torch_gpu, fmt, mtok, n, k, rng):
         e = (0, 60)[i == 1] or (0, -60)[i == mtok - 1]
         chk = check_against_oracle(got[i: i + 1] * np.float32(2.0 ** -e), ref[i: i + 1] * np.float32(2.0 ** -e))
         assert chk.ok() and chk.within, (fmt, mtok, n, k, i, chk)
+
+
+@pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
+@pytest.mark.parametrize("mtok", [3, 8, 13])
+def test_gemv_rowm_tiles_per_workgroup(torch_gpu, fmt, mtok, rng, monkeypatch):
+    """67 tiles as 1 to 9 a workgroup, an uneven last round in each: every tail of the loop with two tiles in flight and
+    of the one with one, and the activation stage reused for the partials: the bits of one tile a workgroup, which lie
+    inside the leaf gate."""
+    from monolith_mi355 import kernels
+    n, k = 1067, 1152
+    m = _matrix(fmt, n, k, rng)
+    x = rbf(rng.standard_normal((mtok, k)).astype(np.float32))
+    w, xd = _upload(torch_gpu, m), to_dev_bf16(torch_gpu, x)
+    outs = {}
+    for rt in (1, 2, 3, 4, 5, 7, 9):
+        monkeypatch.setenv("MI_GEMV_ROWM", f"0,{rt}")
+        launch = _plan(w, xd)
+        assert launch[0] == 3 and launch[3] == rt, launch
+        outs[rt] = kernels.gemv(w, xd, out_f32=True).cpu().numpy()
+        assert np.array_equal(outs[rt].view(np.uint32), outs[1].view(np.uint32)), rt
+    chk = check_against_oracle(outs[1], ON.matmul_acc(x, _dequant(m)))
+    assert chk.ok() and chk.within, (fmt, mtok, chk)
 
 
 @pytest.mark.parametrize("fmt,n,k", [("fp8_e4m3", 170056, 2048), ("nvfp4", 170056, 2048), ("fp8_e4m3", 57352, 6144)])
@@ -458,7 +483,7 @@ def test_gemv_two_tokens(torch_gpu, fmt, big, norm, rng):
 
 @pytest.mark.parametrize("fmt,n,k", [("nvfp4", 12296, 3200), ("nvfp4", 7000, 6144), ("int4_affine", 12296, 3200),
                                      ("fp8_e4m3", 13720, 3136), ("fp8_e4m3", 170056, 3072), ("bf16", 5320, 2080)])
-def test_gemv_two_tokens_norm_in_one_launch(torch_gpu, fmt, n, k):
+def test_gemv_two_tokens_norm_in_one_launch(torch_gpu, fmt, n, k, monkeypatch):
     """Two tokens on gemv_rowm with the input norm fused, over a last slice of one chunk, whole slices up to twelve
     waves, and more tiles than one round of workgroups: the bits of norm_apply and the plain GEMV after it (at a row
     stride past K), of mi_gemv_noalloc, and of a graph captured before any eager call on its stream, replayed with
@@ -486,6 +511,12 @@ def test_gemv_two_tokens_norm_in_one_launch(torch_gpu, fmt, n, k):
         bound = xn.double().abs() @ part.abs().T                 # 32-bit sums of k products: a part of sum |x·w|
         assert ((want[:, lo: lo + 32768].double() - xn.double() @ part.T).abs() <= 2.0 ** -18 * bound).all()
     assert torch.equal(kernels.gemv(w, x, **kw), want)
+    for rt in (1, 2, 3, 4, 5, 7):                                 # every tail of the tile loops
+        monkeypatch.setenv("MI_GEMV_ROWM", f"0,{rt}")
+        launch = _plan(w, x, **kw)
+        assert launch[0] == 3 and launch[3] == rt, launch
+        assert torch.equal(kernels.gemv(w, x, **kw), want), rt
+    monkeypatch.delenv("MI_GEMV_ROWM")
     out = torch.zeros_like(want)
     d, _ = kernels._gemv_desc(w, x, out=out, **kw)
     torch.cuda.synchronize()
@@ -564,7 +595,7 @@ def test_gemv_split_k_fold_in_kernel(torch_gpu):
 @pytest.mark.parametrize("fmt,n,k,mtok,epi,env", [
     ("nvfp4", 5120, 17408, 8, "residual", {}),              # gemv_rowm, K splits: the reduction writes x_next
     ("nvfp4", 5120, 17408, 3, "residual", {}),
-    ("int4_affine", 2048, 8192, 8, "residual", {}),         # gemv_tk splits
+    ("int4_affine", 2048, 8192, 8, "residual", {}),
     ("nvfp4", 1040, 17408, 1, "residual", {"MI_GEMV_FOLD": "0"}),   # gemv_row splits through the reduction launch
     ("nvfp4", 5120, 17408, 1, "residual", {}),              # splits folded in the kernel: a norm launch follows
     ("nvfp4", 2048, 5120, 8, None, {}),                     # one split: a norm launch follows
@@ -573,7 +604,7 @@ def test_gemv_split_k_fold_in_kernel(torch_gpu):
     ("nvfp4", 8200, 12288, 4, "residual", {}),              # wider: the reduction, then a norm launch
     ("nvfp4", 1032, 12288, 16, "residual", {}),             # N not a multiple of 16, sixteen tokens
     ("fp8_e4m3", 5120, 17408, 8, "residual", {}),           # per-row scales applied in the reduction
-    ("bf16", 2048, 8192, 8, None, {}),                      # BF16 weights (gemv_tk)
+    ("bf16", 2048, 8192, 8, None, {}),                      # BF16 weights
 ])
 def test_gemv_next_norm(torch_gpu, fmt, n, k, mtok, epi, env, rng, monkeypatch):
     """``next_norm``: y is bit-identical to the same GEMV without it, and x_next bit-identical to ``norm_apply`` of

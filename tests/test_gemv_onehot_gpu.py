@@ -2,7 +2,7 @@
 no BF16 rounding) is column j of the weight matrix, so every output must equal the oracle's ``dequantize`` bit for
 bit — a single product 1·w and additions of zeros round nothing. This pins the decode each kernel actually runs
 (``gemv_row``'s BF16 pairs with the block scale's mantissa applied once per block, ``gemv_rowp``, the split-K fold, ``gemv_row`` over several token passes,
-``gemv_rowm``'s and ``gemv_tk``'s exact F16 operands on the matrix cores), not only ``mi_dequant``'s, for every
+``gemv_rowm``'s exact F16 or BF16 operands and ``gemv_tk``'s on the matrix cores), not only ``mi_dequant``'s, for every
 weight format (a weight of −0, an E2M1 code, comes out as +0, the sign a sum of zeros has). Ragged N (a partial last tile) and K long enough for three K splits are covered."""
 
 import numpy as np
@@ -61,12 +61,8 @@ def test_one_hot_columns_are_the_dequantized_weights(torch_gpu, fmt, plan, monke
         pytest.skip("gemv_tk has no FP8 path: FP8 runs on gemv_row / gemv_rowm")
     if fmt != "bf16" and plan == "row_passes":
         pytest.skip("the token passes plan takes small BF16 matrices (and grouped NVFP4, tested with the MoE)")
-    if fmt == "bf16" and plan.startswith("rowm"):
-        pytest.skip("gemv_rowm takes NVFP4, FP8 and INT4; BF16 at M >= 3 runs on gemv_tk")
     for key, val in env.items():
         monkeypatch.setenv(key, val)
-    if fmt == "int4_affine" and plan.startswith("rowm"):      # INT4 takes gemv_rowm only when it is pinned
-        monkeypatch.setenv("MI_GEMV_KERNEL", "rowm")
     n = 40
     k = 3072 if "split" in plan else 1024
     rng = np.random.default_rng(abs(hash((fmt, plan))) % 2 ** 32)
