@@ -75,8 +75,7 @@ def upload(specs, device="cuda", row_scales=None) -> PackedWeight:
 
 
 def _bf16_2d(t, name, aligned=True):
-    s = t.stride()
-    if t.dtype != _torch().bfloat16 or len(s) != 2 or s[1] != 1:
+    if t.dtype != _torch().bfloat16 or len(s := t.stride()) != 2 or s[1] != 1:
         raise ValueError(f"{name}: expected a row-major 2-D bfloat16 tensor, got {t.dtype} {tuple(t.shape)}")
     if aligned and (t.data_ptr() % 16 or s[0] % 8):
         raise ValueError(f"{name}: needs 16-byte alignment and a row stride multiple of 8")

@@ -24,6 +24,20 @@ def test_header_declares_entry_points():
     assert {"mi_gemv", "mi_dequant", "mi_malloc", "mi_graph_launch"} <= names
 
 
+def test_wrapper_names_a_wrong_operand():
+    """An array that is no bfloat16 tensor (a NumPy one has no ``stride()``), or one of another shape or layout, is refused
+    with the operand's name, whatever its type offers."""
+    import numpy as np
+    import torch
+
+    from monolith_mi355 import kernels
+    w = kernels.PackedWeight("bf16", 16, 64, 1, torch.zeros(16), None)
+    bf = torch.zeros((2, 64), dtype=torch.bfloat16)
+    for x in (np.zeros((2, 64), np.float32), bf.float(), bf[0], bf.T, torch.zeros((2, 64)).to_sparse()):
+        with pytest.raises(ValueError, match="gemv x"):
+            kernels.gemv(w, x)
+
+
 def test_library_exports_every_declared_symbol():
     from monolith_mi355.runtime import hip
     lib = hip.load()
