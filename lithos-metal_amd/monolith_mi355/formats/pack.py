@@ -78,8 +78,7 @@ def _two_tokens_plan(fmt: str, n: int, k: int, pins) -> int:
     from ..runtime import hip
     out = (C.c_int32 * 7)()
     d = hip.MiGemvDesc(format=hip.MI_FMT[fmt], n=n, k=k, m=2, w=256, x=256, ldx=k, y=256, ldy=n)   # nothing is read
-    hip.call("mi_gemv_plan", C.byref(d), out)
-    return out[0]
+    return 0 if hip.load().mi_gemv_plan(C.byref(d), out) else out[0]     # a matrix that no GEMV takes fails at its launch
 
 
 @dataclass

@@ -212,7 +212,8 @@ def test_emit_without_adjacency_keeps_the_reference_split(tmp_path):
 
 @pytest.mark.parametrize("z_rows,qkv_rows,k,folds", [(6144, 10240, 5120, False),   # 47 MB in all, 17.7 the first slab
                                                        (6144, 640, 5120, True),       # 19.5 MB in all
-                                                       (6144, 10240, 2048, True)])    # a short K
+                                                       (6144, 10240, 2048, True),     # a short K
+                                                       (6144, 10240, 5000, True)])    # no whole chunks: refused at its launch
 def test_conv_fold_at_two_tokens_counts_every_merged_slab(z_rows, qkv_rows, k, folds):
     """At T = 2 the conv folds into the input projection unless its launch, over the rows of all merged slabs, runs on
     the matrix cores."""
