@@ -194,14 +194,18 @@ __device__ __forceinline__ f16x8 int4_decode8(uint32_t dw) {
   return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
-// The same codes as F16 denormals n·2^-24: exact, and seven instructions for eight weights instead of eleven. (Two fewer
-// with the odd nibbles left where they stand, as 16n, cost their activations four binades at the low end.)
-__device__ __forceinline__ f16x8 int4_decode8_denormal(uint32_t dw) {
-  union { uint32_t u[4]; f16x8 h; } p;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) p.u[i] = (dw >> (4 * i)) & 0x000F000Fu;
-  return p.h;
+// The same in seven instructions instead of eleven, in the order int4_byte8: a byte n below 16 is n·2^-9 in FP8 E4M3 (its
+// denormals go on into the first binade). As F16 denormals n·2^-24 (five instructions, no conversion) the codes lose bits
+// on the matrix cores, which align a step's products by the operands' nominal exponents, -14 for every denormal, and cut
+// what lies below: error against 64 bits, 8192 x 5120, 1.7e-6, and 2e-5 where the activations spread over binades,
+// against 1e-7 with normal operands.
+__device__ __forceinline__ f16x8 int4_decode8_bytes(uint32_t dw) {
+  const uint32_t lo = dw & 0x0F0F0F0Fu, hi = (dw >> 4) & 0x0F0F0F0Fu;
+  const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false), h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true);
+  const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false), h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, true);
+  return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
+__device__ __forceinline__ int int4_byte8(int i) { return 2 * (i & 3) + (i >> 2); }   // (n0, n2, n4, n6, n1, n3, n5, n7)
 
 // FP8 E4M3: codes 2j, 2j+1 of a dword (hi: 2, 3) → exact BF16 / F16 pairs (scale 1: the tensor scale is the row's)
 __device__ __forceinline__ bf16x2 cvt_fp8x2_bf16(uint32_t dw, bool hi) {
@@ -1065,9 +1069,9 @@ void gemv_rowp(Args a) {
 // as one is consumed. FP8 and BF16 take BF16 operands instead (their weights
 // are exact BF16, the activations as they are): BF16 8192 x 4096 at M = 3 / 8 / 16 22.3 / 22.5 / 23.2 us on gemv_tk, 13.5 /
 // 14.0 / 14.8 here. A
-// tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to F16
-// denormals n·2^-24, the activations take the codes' column order (int4_perm8) and each 64-column group's dot product is
-// scaled and offset by its (scale, bias) pair with the token's Σx over the group (in the wave's LDS rows).
+// tile's K slices meet in LDS after the last tile, in the gemv_row order. INT4: the codes decode to exact F16
+// integers, the activations take the codes' column order (int4_byte8) and each 64-column group's dot product is scaled
+// and offset by its (scale, bias) pair with the token's Σx over the group (in the wave's LDS rows).
 // LDS: (TWO: Σx² [2][12]) | (INT4: Σx [S][KW][2][16]) | red [S][row_ld floats]: a wave's activation stage, then its [rt][16 tokens][16 rows].
 constexpr int ROWM_SLD = 1024 + 16;             // bytes of a staged activation row (512 columns), padded
 constexpr int ROWM_S = 12;                      // waves at most
@@ -1134,9 +1138,9 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     }
     f16x8 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_perm8(e) : e];      // INT4: the codes' order inside 8 columns
+    for (int e = 0; e < 8; ++e) o[e] = h[I4 ? int4_byte8(e) : e];      // INT4: the codes' order inside 8 columns
     *reinterpret_cast<f16x8*>(stage + r * ROWM_SLD + 16 * lane) = o;
-    return I4 ? pe + 24 : pe;
+    return pe;
   };
   uint4 xr[4], xn[4], xa[KW][SPC];
   float4 w0, w1;
@@ -1199,7 +1203,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
 #pragma unroll
     for (int s = 0; s < SPC; ++s)
       if (TWO || !BA || m_row >= cnt) xa[cc][s] = uint4{0u, 0u, 0u, 0u};
-  int ps[4] = {0, 0, 0, 0};                     // the lane's output tokens are 4g + i: their p (INT4: of the codes' 2^-24 too)
+  int ps[4] = {0, 0, 0, 0};                     // the lane's output tokens are 4g + i: their p
   auto take_rows = [&] {                        // the lane's token from the stage
 #pragma unroll
     for (int cc = 0; cc < KW; ++cc)
@@ -1213,7 +1217,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
     u16x2_t least = {0xFFFF, 0xFFFF};           // of the magnitudes less one: zeros come last
 #pragma unroll
     for (int q = 0; q < 4; ++q) least = __builtin_elementwise_min(least, (u16x2_t)(__builtin_bit_cast(u16x2_t, vv[q] & 0x7FFF7FFFu) - (u16x2_t){1, 1}));
-    return (int)min((uint32_t)least.x, (uint32_t)least.y) + 1 < (p - (I4 ? 24 : 0) + 141 - 31) * 128;
+    return (int)min((uint32_t)least.x, (uint32_t)least.y) + 1 < (p + 141 - 31) * 128;
   };
   if constexpr (TWO) {
     // Two tokens: the fused norm here (one row load, one barrier among the waves), so the call stays one launch without
@@ -1251,7 +1255,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         // A slice that spans more than the 32 binades F16 holds (8-bit values down to 2^-17) takes the operand rows that
         // two tokens leave idle: row 2L + t the values of token t whose exponent lies 32 L to 32 L + 31 below the
         // slice's, by 2^(32 L - p): every value exact, as gemv_row has them. The rows' sums meet in tile_mma
-        const int p[2] = {ps[0] - (I4 ? 24 : 0), ps[1] - (I4 ? 24 : 0)};
+        const int p[2] = {ps[0], ps[1]};
 #pragma unroll 1
         for (int grp = 0; grp < 4; ++grp) {
 #pragma unroll
@@ -1260,7 +1264,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
             f16x8 o;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-              const int src = I4 ? int4_perm8(e) : e;
+              const int src = I4 ? int4_byte8(e) : e;
               const uint32_t bits = (src & 1) ? v[t][src >> 1] >> 16 : v[t][src >> 1] & 0xFFFFu;
               const int d = p[t] + 141 - max((int)(bits & 0x7FFFu) >> 7, 1);   // binades below the slice's exponent
               o[e] = (max(d, 0) >> 5) == lev ? (f16_t)__builtin_amdgcn_ldexpf(bf16_bits_to_f32(bits), 32 * lev - p[t]) : (f16_t)0.0f;
@@ -1312,7 +1316,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
           for (int e = 0; e < 8; ++e) sx += (float)h[e];
         }
         sx = add_xor32(add_xor16(cc < kw ? sx : 0.0f));
-        if (g == 0) sxw[(cc * 2 + gp) * 16 + m_row] = sx * 0x1p-24f;     // in the units of the codes' dot products
+        if (g == 0) sxw[(cc * 2 + gp) * 16 + m_row] = sx;
       }
     wave_lds_sync();
   }
@@ -1338,10 +1342,10 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         }
       } else if constexpr (I4) {                // the two 64-column groups, each scaled and offset on its own
         f32x4 da = {0.f, 0.f, 0.f, 0.f}, db = {0.f, 0.f, 0.f, 0.f};
-        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][0]), int4_decode8_denormal(dw[0]), da, 0, 0, 0);
-        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][1]), int4_decode8_denormal(dw[1]), da, 0, 0, 0);
-        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][2]), int4_decode8_denormal(dw[2]), db, 0, 0, 0);
-        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][3]), int4_decode8_denormal(dw[3]), db, 0, 0, 0);
+        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][0]), int4_decode8_bytes(dw[0]), da, 0, 0, 0);
+        da = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][1]), int4_decode8_bytes(dw[1]), da, 0, 0, 0);
+        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][2]), int4_decode8_bytes(dw[2]), db, 0, 0, 0);
+        db = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, xa[cc][3]), int4_decode8_bytes(dw[3]), db, 0, 0, 0);
         const uint2 sb = sbs[cc];
         const float sca = bf16_bits_to_f32(sb.x & 0xFFFFu), bia = bf16_bits_to_f32(sb.x >> 16);
         const float scb = bf16_bits_to_f32(sb.y & 0xFFFFu), bib = bf16_bits_to_f32(sb.y >> 16);
@@ -1365,7 +1369,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       }
       __builtin_amdgcn_sched_barrier(0);      // decode chunk by chunk: keeps the decoded operands' registers few
     }
-    // the power by v_ldexp: as a float, INT4's 2^(p + 24) need not be finite
+    // the power by v_ldexp, which takes it whatever the slice's magnitude
     float* rp = red + wave * a.row_ld + jt * 256;
     float o[4];
 #pragma unroll
