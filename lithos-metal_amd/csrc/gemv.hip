@@ -1082,6 +1082,7 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   constexpr int SPC = KC / 32;                  // MFMA steps per chunk: the lane's KC/4 columns, 8 per step
   // BA: BF16 operands, the activations as they are (FP8 codes and BF16 weights are exact BF16)
   constexpr bool I4 = FMT == FMT_INT4, BA = FMT == FMT_FP8 || FMT == FMT_BF16;
+  constexpr bool PAIRS = TWO && (FMT == FMT_NVFP4 || FMT == FMT_FP8);   // the sums of two tokens spread over idle rows
   constexpr int UB = I4 ? UNIT_Q : 1024;        // bytes from one chunk's codes to the next
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1242,15 +1243,27 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       for (int t = 0; t < 2; ++t) *reinterpret_cast<uint4*>(stage + t * ROWM_SLD + 16 * lane) = uint4{v[t][0], v[t][1], v[t][2], v[t][3]};
     } else {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {             // 2^p in every lane; the k-group 0 lanes hold the two tokens' outputs
+      for (int t = 0; t < 2; ++t) {             // p in every lane: lane row 4g + i is token i & 1's
         ps[t] = stage_row(t, v[t]);
         wide |= __ballot(below(v[t], ps[t])) != 0;
       }
     }
     wave_lds_sync();
-    if (m_row < 2) take_rows();
+    // NVFP4 and FP8 (no weight is infinite): the operand rows that two tokens leave idle keep the sums short: row 2P + t
+    // holds token t in the slice's MFMA steps 2P and 2P + 1 and zeros in the others, so a row adds up 64 columns and the
+    // rows meet in tile_mma, as a tree. (The whole slice in rows 0 and 1, error against 64 bits at 8192 x 5120: 9.4e-8 and
+    // 1.6e-7; gemv_row 7.9e-8 and 1.3e-7)
+    if constexpr (PAIRS) {
+#pragma unroll
+      for (int st = 0; st < KW * SPC; ++st)
+        if ((m_row >> 1) == (st >> 1))
+          xa[st / SPC][st % SPC] = *reinterpret_cast<const uint4*>(stage + (m_row & 1) * ROWM_SLD + 2 * (st / SPC * KC + xcol(st % SPC)));
+    } else {
+      if (m_row < 2) take_rows();
+    }
     wave_lds_sync();
     if constexpr (!BA) {
+      ps[2] = ps[0]; ps[3] = ps[1];
       if (wide) {
         // A slice that spans more than the 32 binades F16 holds (8-bit values down to 2^-17) takes the operand rows that
         // two tokens leave idle: row 2L + t the values of token t whose exponent lies 32 L to 32 L + 31 below the
@@ -1324,6 +1337,12 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
   // ---- tile by tile: 16 MFMAs over the slice, the partial (tokens × rows) into LDS ----------------------------------
   auto tile_mma = [&](const uint4 (&u)[KW], const uint4 sv, const uint2 (&sbs)[I4 ? KW : 1], int jt) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // BF16 and INT4: several short chains (BF16 one of 16 steps: error against 64 bits 1.3e-7, gemv_tk 0.9e-7 to 2.1e-7,
+    // gemv_row 0.8e-7)
+    constexpr int NC = FMT == FMT_BF16 ? (TWO ? 8 : 4) : I4 ? 2 : 1;
+    f32x4 ch[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) ch[i] = acc;
 #pragma unroll
     for (int cc = 0; cc < KW; ++cc) {
       if (cc >= kw) break;
@@ -1353,12 +1372,12 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
         const f32x4 sxb = *reinterpret_cast<const f32x4*>(sxw + (cc * 2 + 1) * 16 + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          acc[i] = fmaf(sca, da[i], fmaf(bia, sxa[i], acc[i]));
-          acc[i] = fmaf(scb, db[i], fmaf(bib, sxb[i], acc[i]));
+          ch[0][i] = fmaf(sca, da[i], fmaf(bia, sxa[i], ch[0][i]));
+          ch[1][i] = fmaf(scb, db[i], fmaf(bib, sxb[i], ch[1][i]));
         }
       } else if constexpr (FMT == FMT_BF16) {
         const bf16x8 bv = __builtin_bit_cast(bf16x8, u[cc]);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[cc][0]), bv, acc, 0, 0, 0);
+        ch[cc % NC] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[cc][0]), bv, ch[cc % NC], 0, 0, 0);
         continue;                               // no decode: nothing to keep apart
       } else {                                  // FP8: the lane's 16 codes, 8 per step
 #pragma unroll
@@ -1369,13 +1388,20 @@ __global__ __launch_bounds__(768) void gemv_rowm(Args a) {
       }
       __builtin_amdgcn_sched_barrier(0);      // decode chunk by chunk: keeps the decoded operands' registers few
     }
+    if constexpr (NC > 1) {
+#pragma unroll
+      for (int w = NC / 2; w > 0; w /= 2)
+#pragma unroll
+        for (int c = 0; c < w; ++c) ch[c] += ch[c + w];
+      acc = ch[0];
+    }
     // the power by v_ldexp, which takes it whatever the slice's magnitude
     float* rp = red + wave * a.row_ld + jt * 256;
     float o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = active ? (BA ? acc[i] : __builtin_amdgcn_ldexpf(acc[i], ps[i])) : 0.0f;
     if constexpr (TWO) {
-      if (wide) {                               // the two tokens' levels
+      if (PAIRS || wide) {                      // the two tokens' rows
         o[0] = quad16_sum(o[0] + o[2]);
         o[1] = quad16_sum(o[1] + o[3]);
       }

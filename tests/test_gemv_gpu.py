@@ -287,11 +287,13 @@ def test_gemv_rowm_plans(torch_gpu, fmt, mtok, n, k, plan, epi, rng, monkeypatch
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
 @pytest.mark.parametrize("mtok,n", [(2, 8192), (3, 1040), (8, 1040), (16, 1040)])
 @pytest.mark.parametrize("spread", [0.0, 2.0])
-def test_gemv_rowm_sums_in_32_bits(torch_gpu, fmt, mtok, n, spread, rng):
+def test_gemv_rowm_sums_in_32_bits(torch_gpu, fmt, mtok, n, spread, rng, monkeypatch):
     """The FP32 output against 64 bits, on the matrix cores' default routes, for normal activations and ones over several
     binades (exp(2 N)). A value goes through about thirty FP32 additions (16 MFMA steps or groups of a slice, ten slices)
     of sums of up to about twice the result: sqrt(30) roundings of 0.29·2^-23 each come to 2^-21.6 of twice the result's
-    norm at most, an operand that loses bits on the way to far more."""
+    norm at most, an operand that loses bits on the way to far more. Nor is it more than
+    1.25 times the error of the kernel that took such calls before (gemv_row, gemv_tk), whose own spread over thousands of
+    outputs is a few percent."""
     torch, k = torch_gpu, 5120
     w = _upload(torch, _matrix(fmt, n, k, rng))
     from monolith_mi355 import kernels
@@ -299,8 +301,18 @@ def test_gemv_rowm_sums_in_32_bits(torch_gpu, fmt, mtok, n, spread, rng):
     xd = to_dev_bf16(torch, rbf(x.astype(np.float32)))
     assert _plan(w, xd)[0] == 3
     ref = xd.double().cpu() @ kernels.dequant(w).double().cpu().T
-    err = kernels.gemv(w, xd, out_f32=True).double().cpu() - ref
-    assert err.norm() <= 2.0 ** -21.6 * ref.norm(), (err.norm() / ref.norm()).item()
+
+    def error():
+        return ((kernels.gemv(w, xd, out_f32=True).double().cpu() - ref).norm() / ref.norm()).item()
+
+    err = error()
+    assert err <= 2.0 ** -21.6, err
+    if mtok == 2 or fmt != "fp8_e4m3":
+        monkeypatch.setenv("MI_GEMV_KERNEL", "row" if mtok == 2 else "tk")
+        assert _plan(w, xd)[0] == (1 if mtok == 2 else 2)
+        before = error()
+        print(f"{fmt} M={mtok} spread={spread}: {err:.2e}, before {before:.2e}", flush=True)
+        assert err <= 1.25 * before, (err, before)
 
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "int4_affine", "fp8_e4m3", "bf16"])
