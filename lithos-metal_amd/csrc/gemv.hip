@@ -1062,9 +1062,9 @@ void gemv_rowp(Args a) {
 // wave's activations for those chunks stay in VGPRs for the whole launch as the F16 A operands of
 // v_mfma_f32_16x16x32_f16 (token = A row; each token power-of-two scaled into F16 range over the wave's slice;
 // a fused input norm runs as its own launch before, see wants_prenorm; TWO, the instantiation for M = 2, takes it itself,
-// and keeps every activation exact where F16 would not: gate|up at M = 2 20.5 us with that code and without);
+// and keeps every activation exact where F16 would not: no time where no slice needs it);
 // the weights are the B operand, decoded exactly to F16. Each wave
-// keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 23.7 us, two 25.5;
+// keeps two tiles in flight (NVFP4 / FP8; INT4 one: 27B gate|up at M = 8 24.0 us, two measured 1.8 more;
 // BF16 one, its tile is 16 chunks) and issues the next as soon
 // as one is consumed. FP8 and BF16 take BF16 operands instead (their weights
 // are exact BF16, the activations as they are): BF16 8192 x 4096 at M = 3 / 8 / 16 22.3 / 22.5 / 23.2 us on gemv_tk, 13.5 /
@@ -2409,9 +2409,9 @@ bool wants_prenorm(const mi_gemv_desc* d) {
 
 // Two tokens over a large weight stream run on gemv_rowm: gemv_row's dot products for two tokens (VALU) fall behind the
 // stream and normalize both rows in every tile's workgroup; the matrix cores take any M at the price of one, the norm is
-// taken once for a workgroup's tiles. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 41.8 → 21.4 us,
-// without 28.8 → 20.3, in_proj with the norm 23.5 → 14.3, INT4 gate|up 30.1 → 20.6, with the norm 46.0 → 23.0, FP8
-// in_proj 31.3 → 17.4, NVFP4 248320 x 5120 with the norm 248 → 124, BF16 8192 x 4096 17.5 → 12.9. Below, and for a short K
+// taken once for a workgroup's tiles. 27B shapes at M = 2, gemv_row → gemv_rowm: gate|up with the norm 41.5 → 23.1 us,
+// without 28.7 → 21.3, in_proj with the norm 23.9 → 15.6, INT4 gate|up 31.7 → 22.6, with the norm 46.3 → 24.9, FP8
+// in_proj with the norm 31.5 → 17.8, NVFP4 248320 x 5120 with the norm 248 → 124, BF16 8192 x 4096 17.2 → 12.8. Below, and for a short K
 // (few waves share a workgroup's activations), gemv_row won or tied: without the norm N = 34816, K = 1024 / 1536 / 2048 /
 // 3072 7.9 / 9.3 / 10.7 / 16.6 against 8.3 / 9.9 / 10.9 / 14.1 us, INT4 K = 2048 16.0 against 18.2, FP8 4096 x 4096 (16.8
 // MB) 5.9 against 7.2, INT4 4096 x 4096 5.8 against 6.4. A K that gemv_rowm would split (over 6144) stays on gemv_row,
