@@ -2458,6 +2458,29 @@ size_t workspace_need(const mi_gemv_desc* d, const Plan& p) {
   return p.prenorm ? prenorm_offset(d, p) + (size_t)d->m * d->k * sizeof(uint16_t) : split_bytes(d, p);
 }
 
+// M >= 3, tall matrices of a short K: gemv_rowm's workgroups are few waves that take dozens of tiles each, and convert up
+// to 16 rows for them; gemv_tk, where it streams such a matrix without K splits and its workgroups fill the CUs (256 of 256
+// or 970 of 1024, not 262 of 512), is as fast or faster, and needs no scratch either. us, gemv_tk against gemv_rowm, M = 3 /
+// 8 / 16: INT4 131072 x 1664 32.2 / 34.8 / 45.5, 43.0 / 47.0 / 55.6 (at M = 16 in two splits: gemv_rowm's), 248320
+// x 256 18.1 / 19.4 / 23.1, 19.3 / 25.1 / 35.7, 65536 x 512 at M = 16 13.0, 15.4, but 89472 x 3072 39.1 / 41.3 / 49.4, 38.1 / 39.0 / 44.0; BF16 50720 x 128
+// 7.2 / 7.7 / 8.2, 8.0 / 9.4 / 12.9, x 512 12.3 / 12.7 / 13.1, 11.3 / 12.5 / 15.9, 131072 x 1536 64.0 / 63.6 / 65.7, 63.8
+// / 66.2 / 72.9, 248320 x 1536 118 / 118 / 120, 124 / 137 / 153; NVFP4 of no whole slices 131072 x 640 19.2 / 20.4 / 21.7,
+// 15.4 / 18.8 / 26.6, 248320 x 1152 42.8 / 44.9 / 47.2, 49.2 / 58.6 / 79.0.
+bool tk_stays(const mi_gemv_desc* d, const Plan& t, int n_tiles) {
+  const int cu = cu_count(), m = d->m, k = d->k;
+  if (!t.kernel) return false;
+  const int wgs = (n_tiles + t.tb - 1) / t.tb * t.ks, rounds = (wgs + cu - 1) / cu * cu;
+  const bool tall = n_tiles >= 32 * cu, taller = n_tiles > 50 * cu;
+  if (t.ks != 1) return false;
+  if (d->format == FMT_BF16 && k <= 256 && m > 8) return true;
+  if (20 * wgs < (d->format == FMT_BF16 ? 13 : 15) * rounds) return false;
+  if (d->format == FMT_INT4) return k < 3072 && (m > 4 || k > 1024 || taller);
+  if (d->format == FMT_BF16)
+    return k <= 128 || (k <= 256 && (m > 4 || tall)) || (m > 8 && (k < 1024 || (k < 2560 && tall))) || (k < 2560 && taller);
+  // NVFP4, a K of no whole 512-column slices
+  return d->format == FMT_NVFP4 && k % 512 && 10 * wgs >= 9 * rounds && k < 1536 && (m > 12 || (m > 10 && k < 1024) || (k > 1024 && taller));
+}
+
 Plan make_plan_fused(const mi_gemv_desc* d) {
   const int fmt = d->format;
   const int chunks = d->k / chunk_cols(fmt);
@@ -2491,10 +2514,14 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
   }
   // Grouped (MoE) NVFP4 launches at M >= 3: routing spreads the tokens over the experts, so a group holds one or
   // two pairs (the shared expert's group all of them): gemv_row takes them two per workgroup (grid z: the passes)
-  // instead of gemv_tk padding every group to 16 MFMA rows. A BF16 matrix of at most 256 KB the same way, two
-  // tokens per workgroup (64 x 2048 at M = 8 / 16 4.3 / 4.3 us against gemv_rowm's 4.4 / 4.9; the MoE router, 257 x 2048,
-  // 5.0 / 6.0 against 4.4 / 5.1)
-  const bool small = !d->groups && !d->gnorm_w && fmt == FMT_BF16 && (size_t)d->n * d->k * 2 <= (256u << 10);
+  // instead of gemv_tk padding every group to 16 MFMA rows. A small BF16 matrix the same way, two tokens per workgroup:
+  // up to 256 KB, and up to 3 MB (K <= 128: 6) where the tiles are a multiple of four, so that the passes of a tile meet
+  // on one XCD or two and read it from their L2 (M = 8 / 16, us, against gemv_rowm: 64 x 2048 4.3 / 4.3, 4.4 / 4.9; 384 x
+  // 2048 4.5 / 4.5, 4.8 / 5.4; 1024 x 512 3.5 / 3.9, 3.8 / 4.9; 14336 x 128 5.0 / 5.8, 4.9 / 6.8; the MoE router, 257 x
+  // 2048 and 17 tiles, 5.0 / 6.0, 4.4 / 5.1; 1792 x 1024, 3.7 MB, 4.5 / 5.1, 4.0 / 4.5)
+  const size_t bf16_bytes = (size_t)d->n * d->k * 2;
+  const bool small = !d->groups && !d->gnorm_w && fmt == FMT_BF16 &&
+                     (bf16_bytes <= (256u << 10) || (n_tiles % 4 == 0 && bf16_bytes < (d->k <= 128 ? 6u << 20 : 3u << 20)));
   if (rows > 2 && ((d->groups && fmt == FMT_NVFP4) || small) && !pin_tk && !pin_rowm &&
       !(getenv("MI_GEMV_PASSES") && getenv("MI_GEMV_PASSES")[0] == '0')) {       // =0: the earlier plans (A/B)
     Plan p = plan_row(d, fmt, chunks, 2, n_tiles, groups);
@@ -2514,6 +2541,10 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
     if (lean) {
       const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
       if (t.kernel && split_bytes(d, t) < split_bytes(d, p)) return t;
+    }
+    if (p.kernel && !pin_rowm && !getenv("MI_GEMV_ROWM") && p.ks == 1) {
+      const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
+      if (tk_stays(d, t, n_tiles)) return t;
     }
     if (p.kernel) return p;
   }

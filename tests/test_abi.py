@@ -138,6 +138,26 @@ def test_wide_matrices_of_long_k_take_no_scratch(fmt, n, k, ms):
         assert out[0] == 2 and out[4] == 1 and hip.load().mi_gemv_workspace_bytes(C.byref(d)) == 0, (m, list(out))
 
 
+@pytest.mark.parametrize("fmt,n,k,m,kernel", [
+    ("int4_affine", 131072, 1664, 3, 2), ("int4_affine", 65536, 512, 16, 2), ("int4_affine", 248320, 256, 3, 2),
+    ("int4_affine", 131072, 1024, 4, 3), ("int4_affine", 131072, 1664, 16, 3), ("int4_affine", 34816, 2048, 16, 3),
+    ("int4_affine", 50176, 4096, 16, 3), ("bf16", 50720, 128, 3, 2), ("bf16", 50720, 512, 16, 2), ("bf16", 50720, 512, 8, 3),
+    ("bf16", 131072, 1536, 16, 2), ("bf16", 131072, 1536, 8, 3), ("bf16", 248320, 1536, 3, 2), ("bf16", 34816, 2048, 16, 3),
+    ("bf16", 89472, 256, 16, 2), ("nvfp4", 131072, 640, 16, 2), ("nvfp4", 131072, 640, 8, 3), ("nvfp4", 131072, 512, 16, 3),
+    ("nvfp4", 248320, 1152, 5, 2), ("nvfp4", 201088, 640, 16, 3), ("fp8_e4m3", 131072, 640, 16, 3),
+    ("bf16", 384, 2048, 16, 1), ("bf16", 257, 2048, 16, 3), ("bf16", 1792, 1024, 8, 3), ("bf16", 14336, 128, 5, 1),
+    ("bf16", 64, 2048, 8, 1)])
+def test_tall_and_small_matrices_keep_their_kernels(fmt, n, k, m, kernel):
+    """At M >= 3 a tall matrix of a short K stays on gemv_tk where that streams it unsplit on full CUs, and a small BF16
+    matrix in gemv_row's token passes where a tile's passes share an XCD's L2: either side of each line. Neither needs
+    scratch."""
+    from monolith_mi355.runtime import hip
+    out = (C.c_int32 * 7)()
+    d = _desc(hip, format=hip.MI_FMT[fmt], n=n, k=k, m=m, ldx=k, ldy=n)
+    hip.call("mi_gemv_plan", C.byref(d), out)
+    assert out[0] == kernel and out[4] == 1 and hip.load().mi_gemv_workspace_bytes(C.byref(d)) == 0, list(out)
+
+
 def test_gemv_rejects_bad_descriptors_before_launch():
     from monolith_mi355.runtime import hip
     lib = hip.load()
