@@ -2472,7 +2472,9 @@ bool tk_stays(const mi_gemv_desc* d, const Plan& t, int n_tiles) {
   const int wgs = (n_tiles + t.tb - 1) / t.tb * t.ks, rounds = (wgs + cu - 1) / cu * cu;
   const bool tall = n_tiles >= 32 * cu, taller = n_tiles > 50 * cu;
   if (t.ks != 1) return false;
-  if (d->format == FMT_BF16 && k <= 256 && m > 8) return true;
+  // the shortest slices and many rows: whether its workgroups fill the CUs or not (INT4 22528 x 256, 176 workgroups, at M =
+  // 16 8.3 us, gemv_rowm 10.7; BF16 248320 x 256 37.2, 46.9)
+  if (m > 8 && n_tiles >= 4 * cu && ((d->format == FMT_BF16 && k <= 256) || (d->format == FMT_INT4 && k <= 512))) return true;
   if (20 * wgs < (d->format == FMT_BF16 ? 13 : 15) * rounds) return false;
   if (d->format == FMT_INT4) return k < 3072 && (m > 4 || k > 1024 || taller);
   if (d->format == FMT_BF16)

@@ -141,7 +141,8 @@ def test_wide_matrices_of_long_k_take_no_scratch(fmt, n, k, ms):
 @pytest.mark.parametrize("fmt,n,k,m,kernel", [
     ("int4_affine", 131072, 1664, 3, 2), ("int4_affine", 65536, 512, 16, 2), ("int4_affine", 248320, 256, 3, 2),
     ("int4_affine", 131072, 1024, 4, 3), ("int4_affine", 131072, 1664, 16, 3), ("int4_affine", 34816, 2048, 16, 3),
-    ("int4_affine", 50176, 4096, 16, 3), ("bf16", 50720, 128, 3, 2), ("bf16", 50720, 512, 16, 2), ("bf16", 50720, 512, 8, 3),
+    ("int4_affine", 50176, 4096, 16, 3), ("int4_affine", 22528, 256, 10, 2), ("int4_affine", 22528, 256, 8, 3),
+    ("bf16", 50720, 128, 3, 2), ("bf16", 50720, 512, 16, 2), ("bf16", 50720, 512, 8, 3),
     ("bf16", 131072, 1536, 16, 2), ("bf16", 131072, 1536, 8, 3), ("bf16", 248320, 1536, 3, 2), ("bf16", 34816, 2048, 16, 3),
     ("bf16", 89472, 256, 16, 2), ("nvfp4", 131072, 640, 16, 2), ("nvfp4", 131072, 640, 8, 3), ("nvfp4", 131072, 512, 16, 3),
     ("nvfp4", 248320, 1152, 5, 2), ("nvfp4", 201088, 640, 16, 3), ("fp8_e4m3", 131072, 640, 16, 3),
