@@ -86,8 +86,10 @@ __global__ __launch_bounds__(NT) void norm_apply(NormArgs a) {
   }
 }
 
-// a thread per vector, whole waves
-int threads_of(int k) { return std::min(NT, (k / 8 + 63) / 64 * 64); }
+// a thread per vector, whole waves. More rows than CUs share them: half the threads, so that four fit a CU, and the rows
+// past 4096 columns in rounds (1000 rows of 8192 with 1024 / 512 threads 8.0 / 7.0 us, of 8200 9.0 / 7.7, of 5120 6.2 /
+// 6.1; 300 rows 4.4 / 4.3, 5.0 / 4.8, 3.7 / 3.9)
+int threads_of(int k, int t) { return std::min(t > 256 ? NT / 2 : NT, (k / 8 + 63) / 64 * 64); }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -106,7 +108,7 @@ extern "C" int mi_rmsnorm_stat(const mi_norm_desc* d, void* stream) {
   if (int rc = check(d, "mi_rmsnorm_stat")) return rc;
   MI_REQUIRE(d->stat, "mi_rmsnorm_stat: null stat");
   NormArgs a{d->t, d->k, d->ldh, 0, 1, d->h, d->stat, nullptr, nullptr, nullptr, 0.0f};
-  hipLaunchKernelGGL(rmsnorm_stat, dim3(d->t), dim3(threads_of(d->k)), 0, static_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(rmsnorm_stat, dim3(d->t), dim3(threads_of(d->k, d->t)), 0, static_cast<hipStream_t>(stream), a);
   MI_TRY_HIP(hipGetLastError(), "rmsnorm_stat launch");
   return MI_OK;
 }
@@ -117,7 +119,7 @@ extern "C" int mi_norm_apply(const mi_norm_desc* d, void* stream) {
   MI_REQUIRE(d->x && al16(d->x) && d->ldx >= d->k && d->ldx % 8 == 0, "mi_norm_apply: bad output x");
   MI_REQUIRE(!d->stat || d->stat_parts >= 1, "mi_norm_apply: stat_parts >= 1 with a stat");
   NormArgs a{d->t, d->k, d->ldh, d->ldx, d->stat_parts, d->h, nullptr, d->stat, d->w, d->x, d->eps};
-  hipLaunchKernelGGL(norm_apply, dim3(d->t), dim3(threads_of(d->k)), 0, static_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(norm_apply, dim3(d->t), dim3(threads_of(d->k, d->t)), 0, static_cast<hipStream_t>(stream), a);
   MI_TRY_HIP(hipGetLastError(), "norm_apply launch");
   return MI_OK;
 }

@@ -54,6 +54,19 @@ def test_norm_strided_and_partials(torch_gpu):
     assert torch.equal(kernels.norm_apply(h, wd, stat=parts, eps=1e-5), dense)
 
 
+@pytest.mark.parametrize("k", [8, 4096, 4104, 5120, 8192, 8200, 17408])
+def test_norm_of_many_rows_is_the_norm_of_few(torch_gpu, k):
+    """More rows than CUs run with half the threads, wide rows in rounds: the same order of the statistic, the same bits."""
+    torch = torch_gpu
+    from monolith_mi355 import kernels
+    g = torch.Generator(device="cuda").manual_seed(k)
+    h = torch.randn(300, k, device="cuda", generator=g).bfloat16()
+    wd = 1.0 + 0.1 * torch.randn(k, device="cuda", generator=g)
+    few = [h[i:i + 16] for i in range(0, 300, 16)]
+    assert torch.equal(kernels.rmsnorm_stat(h), torch.cat([kernels.rmsnorm_stat(x) for x in few]))
+    assert torch.equal(kernels.norm_apply(h, wd), torch.cat([kernels.norm_apply(x, wd) for x in few]))
+
+
 def test_norm_rejects_bad_shapes(torch_gpu):
     torch = torch_gpu
     from monolith_mi355 import kernels
