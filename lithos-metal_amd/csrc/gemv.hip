@@ -2466,21 +2466,23 @@ size_t workspace_need(const mi_gemv_desc* d, const Plan& p) {
 // 7.2 / 7.7 / 8.2, 8.0 / 9.4 / 12.9, x 512 12.3 / 12.7 / 13.1, 11.3 / 12.5 / 15.9, 131072 x 1536 64.0 / 63.6 / 65.7, 63.8
 // / 66.2 / 72.9, 248320 x 1536 118 / 118 / 120, 124 / 137 / 153; NVFP4 of no whole slices 131072 x 640 19.2 / 20.4 / 21.7,
 // 15.4 / 18.8 / 26.6, 248320 x 1152 42.8 / 44.9 / 47.2, 49.2 / 58.6 / 79.0.
-bool tk_stays(const mi_gemv_desc* d, const Plan& t, int n_tiles) {
+bool tk_may_stay(const mi_gemv_desc* d, int n_tiles) {           // by its sizes: most calls never ask for gemv_tk's plan
   const int cu = cu_count(), m = d->m, k = d->k;
-  if (!t.kernel) return false;
-  const int wgs = (n_tiles + t.tb - 1) / t.tb * t.ks, rounds = (wgs + cu - 1) / cu * cu;
   const bool tall = n_tiles >= 32 * cu, taller = n_tiles > 50 * cu;
-  if (t.ks != 1) return false;
-  // the shortest slices and many rows: whether its workgroups fill the CUs or not (INT4 22528 x 256, 176 workgroups, at M =
-  // 16 8.3 us, gemv_rowm 10.7; BF16 248320 x 256 37.2, 46.9)
-  if (m > 8 && n_tiles >= 4 * cu && ((d->format == FMT_BF16 && k <= 256) || (d->format == FMT_INT4 && k <= 512))) return true;
-  if (20 * wgs < (d->format == FMT_BF16 ? 13 : 15) * rounds) return false;
+  if (n_tiles < 4 * cu) return false;
   if (d->format == FMT_INT4) return k < 3072 && (m > 4 || k > 1024 || taller);
   if (d->format == FMT_BF16)
     return k <= 128 || (k <= 256 && (m > 4 || tall)) || (m > 8 && (k < 1024 || (k < 2560 && tall))) || (k < 2560 && taller);
   // NVFP4, a K of no whole 512-column slices
-  return d->format == FMT_NVFP4 && k % 512 && 10 * wgs >= 9 * rounds && k < 1536 && (m > 12 || (m > 10 && k < 1024) || (k > 1024 && taller));
+  return d->format == FMT_NVFP4 && k % 512 && k < 1536 && (m > 12 || (m > 10 && k < 1024) || (k > 1024 && taller));
+}
+bool tk_stays(const mi_gemv_desc* d, const Plan& t, int n_tiles) {
+  if (!t.kernel || t.ks != 1) return false;
+  // the shortest slices and many rows: whether its workgroups fill the CUs or not (INT4 22528 x 256, 176 workgroups, at M =
+  // 16 8.3 us, gemv_rowm 10.7; BF16 248320 x 256 37.2, 46.9)
+  if (d->m > 8 && ((d->format == FMT_BF16 && d->k <= 256) || (d->format == FMT_INT4 && d->k <= 512))) return true;
+  const int cu = cu_count(), wgs = (n_tiles + t.tb - 1) / t.tb, rounds = (wgs + cu - 1) / cu * cu;
+  return 20 * wgs >= (d->format == FMT_BF16 ? 13 : d->format == FMT_INT4 ? 15 : 18) * rounds;
 }
 
 Plan make_plan_fused(const mi_gemv_desc* d) {
@@ -2544,7 +2546,7 @@ Plan make_plan_fused(const mi_gemv_desc* d) {
       const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
       if (t.kernel && split_bytes(d, t) < split_bytes(d, p)) return t;
     }
-    if (p.kernel && !pin_rowm && !getenv("MI_GEMV_ROWM") && p.ks == 1) {
+    if (p.kernel && p.ks == 1 && tk_may_stay(d, n_tiles) && !pin_rowm && !getenv("MI_GEMV_ROWM")) {
       const Plan t = plan_tk(d, fmt, chunks, n_tiles, groups, rows);
       if (tk_stays(d, t, n_tiles)) return t;
     }
